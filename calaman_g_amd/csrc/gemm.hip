@@ -10,26 +10,24 @@
 // gemm with beta = 1 over it).
 //
 // Kernel shape:
-//   * a BM x BN tile of C per workgroup of NT lanes (NT/64 wave64), each wave
-//     owning a WM x WN sub-tile built from 16 x 16 MFMA tiles
-//     (v_mfma_f64_16x16x4_f64 / v_mfma_f32_16x16x4_f32, 4 accumulator values
-//     per lane);
-//   * K advances in slices of BK, double-buffered in LDS: the next slice is
-//     fetched global -> VGPR while the current one is multiplied, then written
-//     to the other LDS stage; one barrier per slice. The loop body has no
-//     branch (the last slice is peeled), which keeps the accumulators in
-//     registers across iterations;
+//   * a tile of C per workgroup, cut into 16 x 16 MFMA tiles (v_mfma_f64_16x16x4_f64 /
+//     v_mfma_f32_16x16x4_f32, 4 accumulator values per lane), one to four a wave;
+//   * K advances in slices, double-buffered in LDS: later slices are fetched global ->
+//     VGPR while the current one is multiplied, then written to the other LDS stage;
+//     one barrier per slice;
 //   * A is staged as As[k][m] (m contiguous, as it arrives from column-major
-//     memory), B as Bs[n][k] with a row of BK + one 16-byte vector, so the 16
-//     lanes that read one k of B hit 16 distinct bank groups;
+//     memory), B as Bs[n][k] at a pitch of 2 banks (mod 32), so the 16 lanes that read
+//     one k of B hit distinct banks;
 //   * workgroups are renumbered so each of the 8 XCDs (dispatched round robin
 //     on the workgroup id) owns a contiguous run of tiles, walked in groups of
-//     4 tile-rows: the A panels an XCD touches stay in its own L2.
+//     4 tile-rows: the A panels an XCD touches stay in its own L2;
+//   * the tile is chosen per product (launch_product) so that the tiles fill the CUs.
 //
 // MFMA operand layout (16x16x4): A lane l holds A[l%16][l/16], B lane l holds
 // B[l/16][l%16]; D lane l holds column l%16 at rows l/16 + 4r for the FP64
 // instruction and rows 4(l/16) + r for the FP32 one (r = 0..3). The FP64 MFMA
 // accumulates the four k terms of a step in order, as a sequential FMA chain.
+#include "gemm_pipe.hpp"
 #include "gemm_tile.hpp"
 
 namespace clm {
@@ -37,7 +35,8 @@ namespace {
 
 using namespace tile;
 
-template <typename S, int BM, int BN, int WM, int WN, int NT, bool kFast, int BK = kBK>
+// Real products of whole 128 x 128 tiles and whole slices at 16-byte aligned columns.
+template <typename S, int BM, int BN, int WM, int WN, int NT, int BK>
 __global__ void __launch_bounds__(NT)
     rgemm_mfma(const GemmArgs<S> g, const int tiles_m, const int tiles_n) {
   using TL = RTile<S, BM, BN, NT, BK>;
@@ -68,12 +67,12 @@ __global__ void __launch_bounds__(NT)
   V ra[TL::A_V], rb[TL::B_V];
   const int KT = (g.K + BK - 1) / BK;
   if (KT > 0) {
-    rgemm_gload<S, BM, BN, NT, BK, kFast>(g, m0, n0, 0, tid, ra, rb);
+    rgemm_gload<S, BM, BN, NT, BK, true>(g, m0, n0, 0, tid, ra, rb);
     rgemm_sstore<S, BM, BN, NT, BK>(As, Bs, tid, ra, rb);
     __syncthreads();
     for (int kt = 0; kt < KT - 1; ++kt) {
       const int cur = kt & 1;
-      rgemm_gload<S, BM, BN, NT, BK, kFast>(g, m0, n0, (kt + 1) * BK, tid, ra, rb);
+      rgemm_gload<S, BM, BN, NT, BK, true>(g, m0, n0, (kt + 1) * BK, tid, ra, rb);
       // the next slice goes into the other stage half-way through this one, so its
       // LDS writes overlap the other waves' MFMAs instead of idling the CU before
       // the barrier (the k-steps still run in ascending order)
@@ -90,163 +89,157 @@ __global__ void __launch_bounds__(NT)
                                              lane, wm0, wn0, acc);
   }
 
-  // 128 x 128 tiles: the sums go column-major into the free LDS stages and the
-  // whole workgroup writes them out in coalesced column pieces
+  // the sums go column-major into the free LDS stages and the whole workgroup writes
+  // them out in coalesced column pieces
   constexpr int LDT = 128 + 16 / sizeof(S);
-  if constexpr (BM == 128 && BN == 128 && 128 * LDT <= 2 * (TL::A_STAGE + TL::B_STAGE)) {
-    __syncthreads();  // every wave is done with the stages
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          L[(wn0 + j * 16 + (lane & 15)) * LDT + wm0 + i * 16 + Mfma<S>::row(lane, r)] =
-              S(acc[i][j][r]);
-    __syncthreads();
-    lds_tile_epilogue<S, NT / 64, kFast>(g, m0, n0, [&](int c, int r) { return L[c * LDT + r]; });
-  } else {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = m0 + wm0 + i * 16 + Mfma<S>::row(lane, r);
-          const int col = n0 + wn0 + j * 16 + (lane & 15);
-          if (kFast || (row < g.M && col < g.N)) epilogue_store(g, row, col, S(acc[i][j][r]));
-        }
-  }
-}
-
-template <typename C, int BM, int BN, int WM, int WN, int NT, bool kFast, int BK = kBK>
-__global__ void __launch_bounds__(NT)
-    cgemm_mfma(const GemmArgs<C> g, const int tiles_m, const int tiles_n) {
-  using TL = CTile<C, BM, BN, NT, BK>;
-  using S = typename CxReal<C>::type;
-  constexpr int WAVES_M = BM / WM;
-  static_assert((BM / WM) * (BN / WN) == NT / 64, "one wave per WM x WN sub-tile");
-  constexpr int TM = WM / 16, TN = WN / 16;
-
-  __shared__ __attribute__((aligned(16))) S L[2 * TL::STAGE];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  int tm, tn;
-  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int wm0 = (wave % WAVES_M) * WM;
-  const int wn0 = (wave / WAVES_M) * WN;
-
-  typename Mfma<S>::acc cr[TM][TN], ci[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      cr[i][j] = Mfma<S>::zero();
-      ci[i][j] = Mfma<S>::zero();
-    }
-
-  C ra[TL::A_E], rb[TL::B_E];
-  const int KT = (g.K + BK - 1) / BK;
-  if (KT > 0) {
-    cgemm_gload<C, BM, BN, NT, BK, kFast>(g, m0, n0, 0, tid, ra, rb);
-    cgemm_sstore<C, BM, BN, NT, BK>(L, tid, ra, rb);
-    __syncthreads();
-    for (int kt = 0; kt < KT - 1; ++kt) {
-      const int cur = kt & 1;
-      cgemm_gload<C, BM, BN, NT, BK, kFast>(g, m0, n0, (kt + 1) * BK, tid, ra, rb);
-      cgemm_compute<C, BM, BN, WM, WN, NT, BK>(L + cur * TL::STAGE, lane, wm0, wn0, cr, ci);
-      cgemm_sstore<C, BM, BN, NT, BK>(L + (cur ^ 1) * TL::STAGE, tid, ra, rb);
-      __syncthreads();
-    }
-    cgemm_compute<C, BM, BN, WM, WN, NT, BK>(L + ((KT - 1) & 1) * TL::STAGE, lane, wm0, wn0, cr,
-                                             ci);
-  }
-
+  static_assert(BM == 128 && BN == 128 && 128 * LDT <= 2 * (TL::A_STAGE + TL::B_STAGE),
+                "the tile fits the stages");
+  __syncthreads();  // every wave is done with the stages
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm0 + i * 16 + Mfma<S>::row(lane, r);
-        const int col = n0 + wn0 + j * 16 + (lane & 15);
-        if (kFast || (row < g.M && col < g.N))
-          epilogue_store(g, row, col, C{S(cr[i][j][r]), S(ci[i][j][r])});
-      }
+      for (int r = 0; r < 4; ++r)
+        L[(wn0 + j * 16 + (lane & 15)) * LDT + wm0 + i * 16 + Mfma<S>::row(lane, r)] =
+            S(acc[i][j][r]);
+  __syncthreads();
+  lds_tile_epilogue<S, NT / 64, true>(g, m0, n0, [&](int c, int r) { return L[c * LDT + r]; });
+}
+
+// One workgroup tile per workgroup, the operands fetched ahead (gemm_pipe.hpp).
+template <typename T, int BM, int BN, int BK, int WM, int WN, int kAhead>
+__global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64)
+    gemm_piped(const GemmArgs<T> g, const int tiles_m, const int tiles_n) {
+  using SH = pipe::Shape<T, BM, BN, BK, (BM / WM) * (BN / WN) * 64>;
+  __shared__ __attribute__((aligned(16))) pipe::plane_t<T> L[2 * SH::STAGE];
+  int tm, tn;
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  pipe::tile_product<SH, T, WM, WN, kAhead>(g, tm, tn, L);
+}
+
+template <typename T, int BM, int BN, int BK, int WM, int WN, int kAhead>
+hipError_t launch_piped(hipStream_t stream, const GemmArgs<T> &g) {
+  const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
+  hipLaunchKernelGGL((gemm_piped<T, BM, BN, BK, WM, WN, kAhead>), dim3(tiles_m * tiles_n),
+                     dim3((BM / WM) * (BN / WN) * 64), 0, stream, g, tiles_m, tiles_n);
+  return hipGetLastError();
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <int BM, int BN, int NT, int BK, typename Kfast, typename Kgen, typename T>
-hipError_t dispatch(hipStream_t stream, const GemmArgs<T> &g, bool fast_layout, Kfast kfast,
-                    Kgen kgen) {
-  const int tiles_m = (g.M + BM - 1) / BM;
-  const int tiles_n = (g.N + BN - 1) / BN;
-  const bool fast = fast_layout && g.M % BM == 0 && g.N % BN == 0 && g.K % BK == 0;
-  const dim3 grid(tiles_m * tiles_n), block(NT);
-  if (fast) hipLaunchKernelGGL(kfast, grid, block, 0, stream, g, tiles_m, tiles_n);
-  else hipLaunchKernelGGL(kgen, grid, block, 0, stream, g, tiles_m, tiles_n);
-  return hipGetLastError();
+constexpr int kCus = 256;
+
+// The workgroup tile of a product: 32 x 32 (4 waves of one MFMA tile), 64 x 64 (16 such
+// waves) or the large tile (16 waves of 2 x 2 or 2 x 1 MFMA tiles). All three run the
+// same k order, so the choice is speed only: the estimate is the rounds of tiles the
+// 256 CUs take, times the measured time of one tile and k (ns, beyond the launch).
+// A lone 32 x 32 tile per CU has one wave per SIMD and waits on its loads (`one`).
+//
+// Measured per product, before (64 x 64 tiles of 4 waves, one slice ahead, no vector
+// loads at odd orders; 128 x 128 at n >= 2048) -> now, with a four-term block, us:
+//   n       FP64           FP32           complex64      complex128
+//   64      13.3 -> 4.3    11.7 -> 3.5    16.7 -> 5.3    20.4 -> 6.3
+//   333     28.5 -> 9.7    24.0 -> 7.4    41.3 -> 14.0   61.8 -> 20.8
+//   501     38.4 -> 12.8   32.5 -> 9.3    57.8 -> 19.3   95.1 -> 29.3
+//   1000    73.8 -> 42.7   63.7 -> 26.0   104.9 -> 77.0  168.6 -> 134.5
+//   1500    199 -> 153     158 -> 86      427 -> 258     826 -> 503
+//   2000    306 -> 277     199 -> 157     570 -> 513     1104 -> 996
+struct TileCost {
+  int bm, bn;
+  double one, more;
+};
+template <typename T>
+constexpr TileCost kSmall{32, 32, 18.4, 10.8};
+template <>
+constexpr TileCost kSmall<float>{32, 32, 11.0, 6.2};
+template <>
+constexpr TileCost kSmall<zc>{32, 32, 31.0, 18.7};
+template <>
+constexpr TileCost kSmall<zd>{32, 32, 50.0, 36.8};
+template <typename T>
+constexpr TileCost kMedium{64, 64, 38.0, 38.0};
+template <>
+constexpr TileCost kMedium<float>{64, 64, 22.0, 22.0};
+template <>
+constexpr TileCost kMedium<zc>{64, 64, 73.0, 73.0};
+template <>
+constexpr TileCost kMedium<zd>{64, 64, 128.0, 128.0};
+template <typename T>
+constexpr TileCost kLarge{128, 128, 138.0, 138.0};
+template <>
+constexpr TileCost kLarge<float>{128, 128, 73.0, 73.0};
+template <>
+constexpr TileCost kLarge<zc>{128, 128, 268.0, 268.0};
+template <>
+constexpr TileCost kLarge<zd>{128, 64, 243.0, 243.0};
+
+inline double estimate(const TileCost &t, int m, int n) {
+  const long tiles = static_cast<long>((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+  const long rounds = (tiles + kCus - 1) / kCus;
+  return rounds == 1 ? t.one : static_cast<double>(rounds) * t.more;
 }
 
-// Real products: 128 x 128 tiles of 16 waves (32 x 32 each, K slices of 32)
-// once they fill the 256 CUs -- the fastest of the swept FP64 shapes at n = 2048
-// and 4096, 4 waves per SIMD hiding the per-slice barrier; 64 x 64 tiles of
-// 4 waves below that.
-template <typename S>
-hipError_t launch_real(hipStream_t stream, const GemmArgs<S> &g) {
-  if (g.M <= 0 || g.N <= 0) return hipSuccess;
-  constexpr int EV = Mfma<S>::EV;
-  const bool fl = (g.lda % EV == 0) && (g.ldb % EV == 0) && aligned16(g.A) && aligned16(g.B);
-  const long big_tiles = static_cast<long>((g.M + 127) / 128) * ((g.N + 127) / 128);
-  if (big_tiles >= 256)
-    return dispatch<128, 128, 1024, 32>(stream, g, fl,
-                                        rgemm_mfma<S, 128, 128, 32, 32, 1024, true, 32>,
-                                        rgemm_mfma<S, 128, 128, 32, 32, 1024, false, 32>);
-  return dispatch<64, 64, 256, kBK>(stream, g, fl, rgemm_mfma<S, 64, 64, 32, 32, 256, true>,
-                                    rgemm_mfma<S, 64, 64, 32, 32, 256, false>);
+template <typename T>
+hipError_t launch_large(hipStream_t stream, const GemmArgs<T> &g) {
+  if constexpr (std::is_same_v<T, zd>) {
+    // 16 waves of 32 x 16 over slices of 16: 1044 -> 997 us at n = 2048 against 8 waves
+    // of 32 x 32 (twice the waves over the same LDS)
+    return launch_piped<T, 128, 64, 16, 32, 16, 1>(stream, g);
+  } else if constexpr (std::is_same_v<T, double>) {
+    // whole tiles and slices at 16-byte aligned columns: no bounds anywhere and 16-byte
+    // column pieces out of LDS, 280 against 285 us at n = 2048
+    const bool fast = g.M % 128 == 0 && g.N % 128 == 0 && g.K % 32 == 0 && g.lda % 2 == 0 &&
+                      g.ldb % 2 == 0 && aligned16(g.A) && aligned16(g.B);
+    if (fast) {
+      const int tiles_m = g.M / 128, tiles_n = g.N / 128;
+      hipLaunchKernelGGL((rgemm_mfma<double, 128, 128, 32, 32, 1024, 32>),
+                         dim3(tiles_m * tiles_n), dim3(1024), 0, stream, g, tiles_m, tiles_n);
+      return hipGetLastError();
+    }
+    return launch_piped<T, 128, 128, 32, 32, 32, 1>(stream, g);
+  } else {
+    return launch_piped<T, 128, 128, 32, 32, 32, 1>(stream, g);
+  }
 }
 
-// Complex products: 128 x 64 tiles of 8 waves (32 x 32 each) once they fill the
-// CUs, 64 x 64 tiles of 4 waves below that; K slices of 16, double-buffered.
-template <typename C>
-hipError_t launch_complex(hipStream_t stream, const GemmArgs<C> &g) {
+template <typename T>
+hipError_t launch_product(hipStream_t stream, const GemmArgs<T> &g) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
-  const long big_tiles = static_cast<long>((g.M + 127) / 128) * ((g.N + 63) / 64);
-  if (big_tiles >= 256)
-    return dispatch<128, 64, 512, kBK>(stream, g, true, cgemm_mfma<C, 128, 64, 32, 32, 512, true>,
-                                       cgemm_mfma<C, 128, 64, 32, 32, 512, false>);
-  return dispatch<64, 64, 256, kBK>(stream, g, true, cgemm_mfma<C, 64, 64, 32, 32, 256, true>,
-                                    cgemm_mfma<C, 64, 64, 32, 32, 256, false>);
+  const double s = estimate(kSmall<T>, g.M, g.N), m = estimate(kMedium<T>, g.M, g.N),
+               l = estimate(kLarge<T>, g.M, g.N);
+  if (l <= m && l <= s) return launch_large<T>(stream, g);
+  if (m <= s) {
+    constexpr int BK = std::is_same_v<T, float> ? 64 : 32;  // a vector a lane and slice
+    return launch_piped<T, 64, 64, BK, 16, 16, 1>(stream, g);
+  }
+  return launch_piped<T, 32, 32, 32, 16, 16, 2>(stream, g);
 }
 
 }  // namespace
 
 hipError_t launch_gemm_d(hipStream_t stream, const GemmArgs<double> &g) {
-  return launch_real<double>(stream, g);
+  return launch_product<double>(stream, g);
 }
 hipError_t launch_gemm_z(hipStream_t stream, const GemmArgs<zd> &g) {
-  return launch_complex<zd>(stream, g);
+  return launch_product<zd>(stream, g);
 }
 
 template <>
 hipError_t launch_gemm<double>(hipStream_t stream, const GemmArgs<double> &g) {
-  return launch_real<double>(stream, g);
+  return launch_product<double>(stream, g);
 }
 template <>
 hipError_t launch_gemm<float>(hipStream_t stream, const GemmArgs<float> &g) {
-  return launch_real<float>(stream, g);
+  return launch_product<float>(stream, g);
 }
 template <>
 hipError_t launch_gemm<zd>(hipStream_t stream, const GemmArgs<zd> &g) {
-  return launch_complex<zd>(stream, g);
+  return launch_product<zd>(stream, g);
 }
 template <>
 hipError_t launch_gemm<zc>(hipStream_t stream, const GemmArgs<zc> &g) {
-  return launch_complex<zc>(stream, g);
+  return launch_product<zc>(stream, g);
 }
 
 }  // namespace clm

@@ -50,8 +50,10 @@ struct Mfma<float> {
 
 __device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, int &tm, int &tn) {
   const int total = tiles_m * tiles_n;
-  int t = bid;
-  if ((total & 7) == 0) t = (bid & 7) * (total >> 3) + (bid >> 3);
+  // XCD x (workgroups x, x + 8, ...) takes a contiguous run of total / 8 tiles, the
+  // first total % 8 of them one more
+  const int x = bid & 7;
+  const int t = x * (total >> 3) + min(x, total & 7) + (bid >> 3);
   constexpr int G = 4;
   const int per_group = G * tiles_n;
   const int group = t / per_group;
