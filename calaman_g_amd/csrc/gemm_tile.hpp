@@ -21,6 +21,38 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBK = 16;
 
+// A load from / store to device memory through a pointer whose address space the
+// compiler cannot see (the batched kernels read their pointers from descriptors). Left
+// generic these become flat instructions, which also count against the LDS counter: every
+// wait for an LDS operand then waits for the operands being fetched ahead.
+#define CLM_GLOBAL __attribute__((address_space(1)))
+template <typename T>
+__device__ __forceinline__ T gld(const T *p) {
+  if constexpr (std::is_same_v<T, zc>) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    const f2 v = *(const CLM_GLOBAL f2 *)p;
+    return zc{v.x, v.y};
+  } else if constexpr (std::is_same_v<T, zd>) {
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 v = *(const CLM_GLOBAL d2 *)p;
+    return zd{v.x, v.y};
+  } else {
+    return *(const CLM_GLOBAL T *)p;
+  }
+}
+template <typename T>
+__device__ __forceinline__ void gst(T *p, T x) {
+  if constexpr (std::is_same_v<T, zc>) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    *(CLM_GLOBAL f2 *)p = f2{x.re, x.im};
+  } else if constexpr (std::is_same_v<T, zd>) {
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    *(CLM_GLOBAL d2 *)p = d2{x.re, x.im};
+  } else {
+    *(CLM_GLOBAL T *)p = x;
+  }
+}
+
 template <typename S>
 struct Mfma;
 
@@ -74,16 +106,16 @@ __device__ __forceinline__ int exp_tag(int gen, int e) {
 template <typename T>
 __device__ __forceinline__ T epilogue_store(const GemmArgs<T> &g, int row, int col, T acc) {
   T v = ops<T>::mul(g.alpha, acc);
-  if (g.Cin) v = ops<T>::add(v, ops<T>::mul(g.beta, g.Cin[row + (long)col * g.ldcin]));
+  if (g.Cin) v = ops<T>::add(v, ops<T>::mul(g.beta, gld(&g.Cin[row + (long)col * g.ldcin])));
   if (g.nterms > 0) {
     T e = (row == col) ? g.coef[0] : ops<T>::zero();
-    if (g.nterms > 1) e = ops<T>::mad(g.coef[1], g.X1[row + (long)col * g.ldx1], e);
+    if (g.nterms > 1) e = ops<T>::mad(g.coef[1], gld(&g.X1[row + (long)col * g.ldx1]), e);
     for (int t = 2; t < g.nterms; ++t)
-      e = ops<T>::mad(g.coef[t], g.bank[(long)(t - 2) * g.bank_stride + row + (long)col * g.ldbank],
-                      e);
+      e = ops<T>::mad(g.coef[t],
+                      gld(&g.bank[(long)(t - 2) * g.bank_stride + row + (long)col * g.ldbank]), e);
     v = ops<T>::add(v, e);
   }
-  g.C[row + (long)col * g.ldc] = v;
+  gst(&g.C[row + (long)col * g.ldc], v);
   return v;
 }
 
@@ -127,7 +159,7 @@ __device__ __forceinline__ void rgemm_gload(
       S v[EV];
 #pragma unroll
       for (int e = 0; e < EV; ++e)
-        v[e] = (gk < g.K && gm + e < g.M) ? g.A[gm + e + (long)gk * g.lda] : S(0);
+        v[e] = (gk < g.K && gm + e < g.M) ? gld(&g.A[gm + e + (long)gk * g.lda]) : S(0);
       ra[it] = *reinterpret_cast<const V *>(v);
     }
   }
@@ -142,7 +174,7 @@ __device__ __forceinline__ void rgemm_gload(
       S v[EV];
 #pragma unroll
       for (int e = 0; e < EV; ++e)
-        v[e] = (gn < g.N && gk + e < g.K) ? g.B[gk + e + (long)gn * g.ldb] : S(0);
+        v[e] = (gn < g.N && gk + e < g.K) ? gld(&g.B[gk + e + (long)gn * g.ldb]) : S(0);
       rb[it] = *reinterpret_cast<const V *>(v);
     }
   }
@@ -230,14 +262,14 @@ __device__ __forceinline__ void cgemm_gload(const GemmArgs<C> &g, int m0, int n0
   for (int it = 0; it < TL::A_E; ++it) {
     const int e = tid + it * NT;
     const int gm = m0 + e % BM, gk = k0 + e / BM;
-    if (kFast || (gm < g.M && gk < g.K)) ra[it] = g.A[gm + (long)gk * g.lda];
+    if (kFast || (gm < g.M && gk < g.K)) ra[it] = gld(&g.A[gm + (long)gk * g.lda]);
     else ra[it] = ops<C>::zero();
   }
 #pragma unroll
   for (int it = 0; it < TL::B_E; ++it) {
     const int e = tid + it * NT;
     const int gk = k0 + e % BK, gn = n0 + e / BK;
-    if (kFast || (gk < g.K && gn < g.N)) rb[it] = g.B[gk + (long)gn * g.ldb];
+    if (kFast || (gk < g.K && gn < g.N)) rb[it] = gld(&g.B[gk + (long)gn * g.ldb]);
     else rb[it] = ops<C>::zero();
   }
 }
@@ -478,17 +510,56 @@ __device__ __forceinline__ void epilogue_put(E *sumt, int p0, int lane, int wm0,
             value(i, j, r);
 }
 
+// Up to 4 elements a lane and round, every term's reads of a round issued together (one
+// element at a time waits for memory once a term and element: 1024 complex64 of order
+// 112, 1.17 -> 1.08 ms); 8 would cost the small tiles a wave of occupancy (1.26 ms).
 template <typename E, int BM, int PW, int NT>
 __device__ __forceinline__ void epilogue_drain(const GemmArgs<E> &g, const E *sumt, int m0,
                                                int c0) {
-  for (int e = threadIdx.x; e < BM * PW; e += NT) {
-    const int r = e % BM, c = e / BM;
-    const int row = m0 + r, col = c0 + c;
-    if (row < g.M && col < g.N) epilogue_store(g, row, col, sumt[c * (BM + 1) + r]);
+  using O = ops<E>;
+  constexpr int PER = BM * PW / NT, kU = (sizeof(E) == 16 ? 2 : 4) / (NT >= 1024 && sizeof(E) > 4 ? 2 : 1);
+  constexpr int U = PER < kU ? PER : kU;
+  static_assert(PER * NT == BM * PW && PER % U == 0 && NT % BM == 0, "the pass splits into rounds");
+  // a lane keeps one row; its columns are NT / BM apart
+  const int r = threadIdx.x % BM, row = m0 + r;
+  if (row >= g.M) return;
+  for (int c = threadIdx.x / BM; c < PW; c += U * (NT / BM)) {
+    E v[U], x[U];
+    auto each = [&](auto f) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) f(u, c0 + c + u * (NT / BM));
+    };
+    auto read = [&](const E *X, long ld) {
+      each([&](int u, int col) {
+        if (col < g.N) x[u] = gld(&X[row + (long)col * ld]);
+      });
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      v[u] = O::mul(g.alpha, sumt[(c + u * (NT / BM)) * (BM + 1) + r]);
+      x[u] = O::zero();
+    }
+    if (g.Cin) {
+      read(g.Cin, g.ldcin);
+      each([&](int u, int) { v[u] = O::add(v[u], O::mul(g.beta, x[u])); });
+    }
+    if (g.nterms > 0) {
+      E s[U];
+      const E z0 = g.coef[0];
+      each([&](int u, int col) { s[u] = row == col ? z0 : O::zero(); });
+      for (int t = 1; t < g.nterms; ++t) {
+        if (t == 1) read(g.X1, g.ldx1);
+        else read(g.bank + (long)(t - 2) * g.bank_stride, g.ldbank);
+        const E ct = g.coef[t];
+        each([&](int u, int) { s[u] = O::mad(ct, x[u], s[u]); });
+      }
+      each([&](int u, int) { v[u] = O::add(v[u], s[u]); });
+    }
+    each([&](int u, int col) {
+      if (col < g.N) gst(&g.C[row + (long)col * g.ldc], v[u]);
+    });
   }
 }
 
-// C = A*B (+ epilogue of g) over the whole n x n output, tile by tile, by all
-// 256 lanes; ends with a barrier, so C is complete for every lane afterwards.
 }  // namespace tile
 }  // namespace clm
