@@ -244,14 +244,18 @@ clm_status_t clm_getrs_z(clm_ctx *ctx, clm_stream_t stream, int n, int nrhs,
  * calaman::expm_herm<T> (src/expm/expm_herm.cppm:145-199): only the uplo triangle of A
  * is read (the other assumed to mirror it; the diagonal's imaginary part ignored),
  * A = U diag(w) U^H, exp(A) = U diag(exp(w)) U^H. The reference takes the
- * eigendecomposition from the vendor syevd / heevd; this library's is a blocked
- * two-sided Jacobi method on the device (off-diagonal Frobenius norm driven below
- * u ||A||_F). uplo: CLM_FILL_MODE_LOWER / CLM_FILL_MODE_UPPER (the BLAS fill-mode
+ * eigendecomposition from the vendor syevd / heevd. Here, up to ||A||_1 = 32, exp(A) is
+ * the library's Taylor exponential of the mirrored matrix, shifted by its mean eigenvalue
+ * and in double (faster and no less accurate there); beyond, for a diagonal A and in a
+ * workspace of the Jacobi blocks alone, a blocked two-sided Jacobi method on the device
+ * (off-diagonal Frobenius norm driven below u ||A||_F). uplo: CLM_FILL_MODE_LOWER / CLM_FILL_MODE_UPPER (the BLAS fill-mode
  * values). dInfo (device int, may be NULL): 0, or 1 when the Jacobi sweeps did not
- * converge within 30 (the result is still written). Synchronizes once per sweep.
+ * converge within 30 (the result is still written). Synchronizes (the norm, then the
+ * exponential's norms or once per sweep).
  * Bad arguments: CLM_STATUS_INVALID_VALUE; a short workspace: CLM_STATUS_ALLOC_FAILED.
- * expm_herm_bufferSize<T> (:97-109): clm_expm_herm_buffer_size_* (three blocks of
- * order n rounded up to 64, where the reference holds two and the solver's scratch). */
+ * expm_herm_bufferSize<T> (:97-109): clm_expm_herm_buffer_size_* (the larger of the
+ * routes' needs; the Jacobi route's own, three blocks of order n rounded up to 64, is
+ * accepted too. The reference holds two blocks and the solver's scratch). */
 #define CLM_FILL_MODE_LOWER 0
 #define CLM_FILL_MODE_UPPER 1
 clm_status_t clm_expm_herm_buffer_size_s(int n, size_t *bytes);

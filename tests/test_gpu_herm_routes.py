@@ -1,0 +1,80 @@
+"""GPU: expm_herm's two routes -- the shifted Taylor exponential up to ||A||_1 = 32, the
+Jacobi sweeps beyond it, for diagonal matrices and in a workspace of the sweeps' size.
+
+Both against numpy's eigh (the oracle). Tolerance: eigh's own normwise error bound
+p(n) u ||A||_2 times exp's condition for a Hermitian matrix (1 + ||A||_2), with p(n) = 8 n:
+well under the 1e-12 the route is held to elsewhere.
+"""
+import numpy as np
+import pytest
+import torch
+
+import calaman_g_amd as cg
+import oracle.herm as oh
+
+pytestmark = pytest.mark.gpu
+
+
+def _spectrum(n, cplx, kind, norm, seed):
+    rng = np.random.default_rng(seed)
+    g = rng.standard_normal((n, n)) + (1j * rng.standard_normal((n, n)) if cplx else 0)
+    if kind == "negative":
+        h = -(g @ g.conj().T)
+    elif kind == "outlier":
+        q, _ = np.linalg.qr(g)
+        w = 0.1 * rng.standard_normal(n)
+        w[0] = -30.0
+        h = (q * w) @ q.conj().T
+    else:
+        h = g
+    h = (h + h.conj().T) / 2
+    return h * (norm / np.abs(h).sum(0).max())
+
+
+def _run(a, uplo, dev, nbytes=None):
+    n, ld = a.shape[0], a.shape[0] + 1
+    dt = torch.complex128 if np.iscomplexobj(a) else torch.float64
+    buf = np.full((n, ld), np.nan, dtype=a.dtype)
+    buf[:, :n] = a.T
+    other = np.tril(np.ones((n, n), bool), -1) if uplo == "U" else np.triu(np.ones((n, n), bool), 1)
+    buf[:, :n].T[other] = np.nan  # never read
+    da = torch.from_numpy(buf).to(dev)
+    de = torch.full((n, ld), 7.0, dtype=dt, device=dev)
+    size = cg.expm_herm_buffer_size(n, dt) if nbytes is None else nbytes
+    work = torch.empty(size, dtype=torch.uint8, device=dev)
+    info = torch.full((1,), -3, dtype=torch.int32, device=dev)
+    assert cg.expm_herm_cm(uplo, n, da, ld, de, ld, work, info) == 0
+    assert int(info.item()) == 0
+    out = de.cpu().numpy()
+    assert np.all(out[:, n:] == 7.0)
+    return out[:, :n].T
+
+
+def _jacobi_bytes(n, size):
+    """the sweeps' blocks: three of order n rounded up to 64, the rotations and the scalars"""
+    up = lambda v: -(-v // 256) * 256
+    np_, k = -(-n // 64) * 64, -(-n // 64)
+    return 3 * up(np_ * np_ * size) + up(k * 4096 * size) + up(4 * k) + 2 * 256 + up(8 * np_)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("kind", ["full", "negative", "outlier"])
+@pytest.mark.parametrize("n,norm", [(1, 3.0), (2, 31.9), (33, 31.9), (33, 32.1), (130, 8.0),
+                                    (130, 60.0)])
+def test_routes_agree_with_eigh(dev, cplx, kind, n, norm):
+    a = _spectrum(n, cplx, kind, norm, 17 * n + int(norm))
+    for uplo, code in (("U", oh.UPPER), ("L", oh.LOWER)):
+        ref = oh.expm_herm(a, code)
+        err = np.linalg.norm(_run(a, uplo, dev) - ref) / np.linalg.norm(ref)
+        assert err <= 8 * n * 1.2e-16 * (1 + np.linalg.norm(a, 2)) + 1e-14
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+def test_a_workspace_of_the_sweeps_size_still_serves(dev, cplx):
+    n = 128
+    a = _spectrum(n, cplx, "full", 4.0, 5)
+    nbytes = _jacobi_bytes(n, 16 if cplx else 8)
+    assert nbytes < cg.expm_herm_buffer_size(n, torch.complex128 if cplx else torch.float64)
+    ref = oh.expm_herm(a)
+    err = np.linalg.norm(_run(a, "U", dev, nbytes) - ref) / np.linalg.norm(ref)
+    assert err <= 1e-12
