@@ -5,14 +5,14 @@
 // Recursive LU (the column split of LAPACK's ?getrf2): factor the left half of
 // a block column, interchange and solve its right half against the unit-lower
 // triangle, subtract the product from the trailing rows, factor the right half.
-// The large updates are the library's MFMA products; the recursion stops at
-// leaf block columns of up to 32 columns whose whole height fits the LDS
-// (128 KiB: 2048 FP64 rows at 8 columns, 4096 at 4, ...), factored by one
-// 1024-lane workgroup in LDS -- pivot search by a (value, index) reduction over
-// every lane, the interchange, the scaling and the rank-1 update of the leaf's
-// remaining columns -- so a leaf costs one load and one store of its rows. Taller
-// leaves (past 16384 FP64 rows) run the same steps on the matrix in memory.
-// The leaf's interchanges are applied at once to every other column of the
+// The large updates are the library's MFMA products; the recursion stops at panels of up
+// to 32 columns and 128 KiB, factored by one 512-lane workgroup with its rows in
+// registers: the pivot search is a shuffle reduction over the waves, and the pivot row
+// reaches every lane through LDS and scalar registers, two barriers a column. A panel
+// waits on that chain of steps, not on arithmetic; 1000 x 16 in FP64 takes 30 us (76 us
+// with the block in LDS, its columns walked by strided lanes, five barriers a column).
+// Panels too tall for the registers run the same steps on the matrix in memory.
+// A panel's interchanges are applied at once to every other column of the
 // matrix, which gives the same matrix as LAPACK's deferred application: the
 // columns to the right are not touched in between, those to the left are final.
 //
@@ -31,8 +31,9 @@ namespace clm {
 namespace {
 
 constexpr int kLeafThreads = 1024;
-constexpr size_t kLeafLdsBytes = 131072;
-constexpr int kLeafMaxCols = 32;
+constexpr int kPanelCols = 32;
+constexpr int kPanelThreads = 512;  // half the waves of 1024 lanes, each sending a pivot row's
+                                    // columns to twice the rows
 constexpr int kTrsmNb = 64;  // triangle order solved in LDS
 
 // i?amax's measure: |x| for real, |re| + |im| for complex
@@ -45,6 +46,18 @@ __device__ inline double sub(double a, double b) { return a - b; }
 __device__ inline float sub(float a, float b) { return a - b; }
 __device__ inline zd sub(zd a, zd b) { return zd{a.re - b.re, a.im - b.im}; }
 __device__ inline zc sub(zc a, zc b) { return zc{a.re - b.re, a.im - b.im}; }
+
+// a - x y, two roundings a component at most
+__device__ inline double msub(double a, double x, double y) { return __builtin_fma(-x, y, a); }
+__device__ inline float msub(float a, float x, float y) { return __builtin_fmaf(-x, y, a); }
+__device__ inline zd msub(zd a, zd x, zd y) {
+  return zd{__builtin_fma(x.im, y.im, __builtin_fma(-x.re, y.re, a.re)),
+            __builtin_fma(-x.im, y.re, __builtin_fma(-x.re, y.im, a.im))};
+}
+__device__ inline zc msub(zc a, zc x, zc y) {
+  return zc{__builtin_fmaf(x.im, y.im, __builtin_fmaf(-x.re, y.re, a.re)),
+            __builtin_fmaf(-x.im, y.re, __builtin_fmaf(-x.re, y.im, a.im))};
+}
 
 __device__ inline double cdiv(double a, double b) { return a / b; }
 __device__ inline float cdiv(float a, float b) { return a / b; }
@@ -71,8 +84,8 @@ __device__ inline double min_normal() {
   return std::is_same_v<real_t<T>, float> ? 1.17549435e-38 : 2.2250738585072014e-308;
 }
 
-// ---- the leaf: a block column of m rows and w <= 32 columns -------------------------------
-// P: the block (LDS copy, leading dimension ldp = m, or the matrix itself). row0 is
+// ---- the panel in memory: a block column of m rows and w columns ----------------------------
+// P: the block, in the matrix itself. row0 is
 // the global row (and column) of the block's first row; ipiv and info get global
 // 1-based indices.
 template <typename T>
@@ -158,23 +171,135 @@ __device__ void leaf_factor(T *P, long ldp, int m, int w, int row0, int *ipiv, i
   }
 }
 
-// the block A[row0 : n, row0 : row0 + w] copied into LDS, factored, copied back
-template <typename T>
-__global__ void __launch_bounds__(kLeafThreads)
-    leaf_lds_kernel(int n, T *A, long lda, int row0, int w, int *ipiv, int *info) {
-  __shared__ __attribute__((aligned(16))) char buf[kLeafLdsBytes];
-  __shared__ double red_v[kLeafThreads / 64];
-  __shared__ int red_i[kLeafThreads / 64 + 1];
-  __shared__ T pivot;
-  T *P = reinterpret_cast<T *>(buf);
+// lane l's value in every lane (l uniform)
+__device__ inline float from_lane(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ inline double from_lane(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane(static_cast<int>(b & 0xffffffffll), l);
+  const int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), l);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) | lo);
+}
+__device__ inline zc from_lane(zc v, int l) { return zc{from_lane(v.re, l), from_lane(v.im, l)}; }
+__device__ inline zd from_lane(zd v, int l) { return zd{from_lane(v.re, l), from_lane(v.im, l)}; }
+
+// The pivot measure as an integer that orders like it: the bits of a non-negative double,
+// -1 for a NaN (below every number), -2 for no row
+__device__ inline long long measure_key(double v) {
+  return v == v ? __double_as_longlong(v) : -1ll;
+}
+// the largest key over a group of `width` lanes and the smallest index that has it
+template <int width>
+__device__ inline void group_argmax(long long &key, int &idx) {
+  long long m = key;
+#pragma unroll
+  for (int off = width / 2; off > 0; off >>= 1) {
+    const long long o = __shfl_xor(m, off);
+    m = o > m ? o : m;
+  }
+  unsigned long long has = __ballot(key == m);
+  if constexpr (width < 64) has &= (1ull << width) - 1;  // the keys repeat past the group
+  if (m == -2) has = 0;  // no row in the group
+  int first = INT_MAX;
+  while (has) {
+    first = min(first, __builtin_amdgcn_readlane(idx, __ffsll(has) - 1));
+    has &= has - 1;
+  }
+  key = m;
+  idx = first;
+}
+
+// the panel A[row0 : n, row0 : row0 + w], w <= W, in registers: lane t holds rows t, t +
+// 512, ... (R of them). leaf_factor's steps and arithmetic; the interchanges of the
+// panel's own earlier columns are left to laswp_kernel. The current column is always
+// register 0: the update writes column c's result to register c - 1, so the steps are one
+// loop (unrolled over the columns they are 64 KB of code run once, and the panel waited
+// for its instructions: 88 us for 1000 x 32). A finished column of L and row of U go
+// straight to memory.
+template <typename T, int W, int R>
+__global__ void __launch_bounds__(kPanelThreads)
+    panel_kernel(int n, T *A, long lda, int row0, int w, int *ipiv, int *info) {
+  constexpr int kWaves = kPanelThreads / 64;
+  // two sets by the column's parity: a set is rewritten two barriers after its last read
+  __shared__ long long red_k[2][kWaves];
+  __shared__ int red_i[2][kWaves];
+  __shared__ T rows[2][2][W];  // the pivot row, and row j that it changes places with
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = n - row0;
   T *blk = A + row0 + static_cast<long>(row0) * lda;
-  for (int c = 0; c < w; ++c)
-    for (int i = threadIdx.x; i < m; i += kLeafThreads) P[i + c * m] = blk[i + c * lda];
-  __syncthreads();
-  leaf_factor<T>(P, m, m, w, row0, ipiv, info, red_v, red_i, &pivot);
-  for (int c = 0; c < w; ++c)
-    for (int i = threadIdx.x; i < m; i += kLeafThreads) blk[i + c * lda] = P[i + c * m];
+  T a[R][W];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      const int i = tid + kPanelThreads * r;
+      a[r][c] = (i < m && c < w) ? blk[i + c * lda] : ops<T>::zero();
+    }
+#pragma unroll 1
+  for (int j = 0; j < w; ++j) {
+    const int set = j & 1;
+    long long key = -2;
+    int bi = INT_MAX;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = tid + kPanelThreads * r;
+      const long long k = measure_key(cabs1(a[r][0]));
+      if (i >= j && i < m && k > key) {  // rows ascend: the first maximum stays
+        key = k;
+        bi = i;
+      }
+    }
+    group_argmax<64>(key, bi);
+    if (lane == 0) {
+      red_k[set][wave] = key;
+      red_i[set][wave] = bi;
+    }
+    __syncthreads();
+    key = red_k[set][lane % kWaves];
+    bi = red_i[set][lane % kWaves];
+    group_argmax<kWaves>(key, bi);
+    const bool nonzero = key != 0;  // a zero pivot: no interchange, no scaling
+    const int p = nonzero ? bi : j;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = tid + kPanelThreads * r;
+      if (i == p) {
+#pragma unroll
+        for (int c = 0; c < W; ++c) rows[set][0][c] = a[r][c];
+      }
+      if (i == j) {
+#pragma unroll
+        for (int c = 0; c < W; ++c) rows[set][1][c] = a[r][c];
+      }
+    }
+    if (tid == 0) {
+      ipiv[row0 + j] = row0 + bi + 1;
+      if (!nonzero) atomicMin(info, row0 + j + 1);
+    }
+    __syncthreads();
+    // lane c of every wave takes column c of the two rows; a column's value then goes to
+    // all lanes through a scalar register
+    const T prow = rows[set][0][lane % W], jrow = rows[set][1][lane % W];
+    if (tid < w - j) blk[j + static_cast<long>(j + tid) * lda] = prow;
+    const T pv = from_lane(prow, 0);
+    const bool safe = cabs1(pv) >= min_normal<T>();
+    const T rp = safe ? cdiv(ops<T>::from_real(1.0), pv) : ops<T>::zero();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = tid + kPanelThreads * r;
+      if (i == p && p != j) {
+#pragma unroll
+        for (int c = 0; c < W; ++c) a[r][c] = from_lane(jrow, c);
+      }
+      T l = a[r][0];
+      if (nonzero) l = safe ? ops<T>::mul(l, rp) : cdiv(l, pv);
+      if (i > j && i < m) blk[i + static_cast<long>(j) * lda] = l;
+#pragma unroll
+      for (int c = 1; c < W; ++c) a[r][c - 1] = sub(a[r][c], ops<T>::mul(l, from_lane(prow, c)));
+      a[r][W - 1] = ops<T>::zero();
+    }
+  }
 }
 
 // the same steps on the matrix in memory, for blocks taller than the LDS holds
@@ -188,15 +313,17 @@ __global__ void __launch_bounds__(kLeafThreads)
                  red_v, red_i, &pivot);
 }
 
-// rows k and ipiv[k] - 1 interchanged for k = k0 .. k1-1 in order, in every column
-// c < ncols outside [skip0, skip1): one lane a column
+// rows k and ipiv[k] - 1 interchanged for k = k0 .. k1-1 in order, in every column c <
+// ncols; in the columns of own0 .. own1-1 none (done) or only those past the column's own
+// (a panel whose kernel left those): one lane a column
 template <typename T>
 __global__ void __launch_bounds__(256)
-    laswp_kernel(int ncols, T *A, long lda, const int *ipiv, int k0, int k1, int skip0, int skip1) {
+    laswp_kernel(int ncols, T *A, long lda, const int *ipiv, int k0, int k1, int own0, int own1,
+                 bool own_done) {
   const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= ncols || (c >= skip0 && c < skip1)) return;
+  if (c >= ncols) return;
   T *col = A + static_cast<long>(c) * lda;
-  for (int k = k0; k < k1; ++k) {
+  for (int k = (c < own0 || c >= own1) ? k0 : own_done ? k1 : c + 1; k < k1; ++k) {
     const int p = ipiv[k] - 1;
     if (p != k) {
       const T t = col[k];
@@ -214,40 +341,68 @@ __global__ void finish_info_kernel(int *info) {
   if (threadIdx.x == 0 && *info == INT_MAX) *info = 0;
 }
 
-// ---- triangular solves: X = T^-1 B, T of order nb <= 64 in LDS ----------------------------------
+// ---- triangular solves: X = T^-1 B, T of order nb <= 64 -------------------------------------
+__device__ inline bool finite(double x) { return isfinite(x); }
+__device__ inline bool finite(float x) { return isfinite(x); }
+__device__ inline bool finite(zd x) { return isfinite(x.re) && isfinite(x.im); }
+__device__ inline bool finite(zc x) { return isfinite(x.re) && isfinite(x.im); }
+
+constexpr int kTrsmWaves = 4;  // waves a workgroup: they share the triangle in LDS
+constexpr int kTrsmCols = 4;   // right-hand sides a wave
+
 // lower = true: T unit lower (forward substitution); false: T upper with its diagonal
-// (backward). One lane a right-hand side, 64 columns a workgroup.
+// (backward). A lane is a row and a wave holds four right-hand sides in registers: step k
+// sends row k's value to every lane and subtracts its column of T, so a solve is nb
+// multiply-adds deep. (A lane a right-hand side, the rows in LDS, is nb^2 / 2 deep: 46 us
+// for nb = 64 however few the columns, now 12 us lower and 24 us upper.) The division by the diagonal is a
+// product with its reciprocal and one correction step; the quotient itself where that is
+// not finite.
 template <typename T, bool kLower>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64 * kTrsmWaves)
     trsm_small_kernel(int nb, int ncols, const T *Tm, long ldt, T *B, long ldb) {
-  __shared__ T tri[kTrsmNb][kTrsmNb + 1];
-  __shared__ T xs[kTrsmNb][kTrsmNb + 1];  // xs[col][row]
-  const int lane = threadIdx.x;
-  const int c0 = blockIdx.x * 64;
-  for (int j = 0; j < nb; ++j)
-    if (lane < nb) tri[lane][j] = Tm[lane + static_cast<long>(j) * ldt];  // tri[row][col]
-  const int nc = min(64, ncols - c0);
-  for (int c = 0; c < nc; ++c)
-    if (lane < nb) xs[c][lane] = B[lane + static_cast<long>(c0 + c) * ldb];
+  __shared__ T tri[kTrsmNb][kTrsmNb + 1];  // tri[k][i]: column k
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int e = tid; e < kTrsmNb * kTrsmNb; e += 64 * kTrsmWaves) {
+    const int i = e % kTrsmNb, k = e / kTrsmNb;
+    tri[k][i] = (i < nb && k < nb) ? Tm[i + static_cast<long>(k) * ldt] : ops<T>::zero();
+  }
+  const int c0 = (blockIdx.x * kTrsmWaves + wave) * kTrsmCols;
+  T x[kTrsmCols];
+#pragma unroll
+  for (int c = 0; c < kTrsmCols; ++c)
+    x[c] = (lane < nb && c0 + c < ncols) ? B[lane + static_cast<long>(c0 + c) * ldb]
+                                         : ops<T>::zero();
   __syncthreads();
-  if (lane < nc) {
-    if (kLower) {
-      for (int i = 1; i < nb; ++i) {
-        T acc = xs[lane][i];
-        for (int j = 0; j < i; ++j) acc = sub(acc, ops<T>::mul(tri[i][j], xs[lane][j]));
-        xs[lane][i] = acc;
+  const T diag = kLower ? ops<T>::from_real(1.0) : tri[lane][lane];
+  const T rdiag = kLower ? diag : cdiv(ops<T>::from_real(1.0), diag);
+#pragma unroll 4
+  for (int s = 0; s < nb; ++s) {
+    const int k = kLower ? s : nb - 1 - s;
+    const T t = tri[k][lane];
+    const bool below = kLower ? lane > k : lane < k;
+    T dk = diag, rk = rdiag;
+    if constexpr (!kLower) {
+      dk = from_lane(diag, k);
+      rk = from_lane(rdiag, k);
+    }
+#pragma unroll
+    for (int c = 0; c < kTrsmCols; ++c) {
+      T xk = from_lane(x[c], k);
+      if constexpr (!kLower) {
+        const T num = xk;
+        T q = ops<T>::mul(num, rk);
+        q = ops<T>::add(q, ops<T>::mul(msub(num, q, dk), rk));
+        if (!finite(q)) q = cdiv(num, dk);
+        xk = q;
+        if (lane == k) x[c] = q;
       }
-    } else {
-      for (int i = nb - 1; i >= 0; --i) {
-        T acc = xs[lane][i];
-        for (int j = i + 1; j < nb; ++j) acc = sub(acc, ops<T>::mul(tri[i][j], xs[lane][j]));
-        xs[lane][i] = cdiv(acc, tri[i][i]);
-      }
+      const T y = sub(x[c], ops<T>::mul(t, xk));
+      if (below) x[c] = y;
     }
   }
-  __syncthreads();
-  for (int c = 0; c < nc; ++c)
-    if (lane < nb) B[lane + static_cast<long>(c0 + c) * ldb] = xs[c][lane];
+#pragma unroll
+  for (int c = 0; c < kTrsmCols; ++c)
+    if (lane < nb && c0 + c < ncols) B[lane + static_cast<long>(c0 + c) * ldb] = x[c];
 }
 
 template <typename T>
@@ -277,7 +432,9 @@ template <typename T, bool kLower>
 hipError_t trsm(hipStream_t st, int nb, int ncols, const T *Tm, long ldt, T *B, long ldb) {
   if (nb <= 0 || ncols <= 0) return hipSuccess;
   if (nb <= kTrsmNb) {
-    trsm_small_kernel<T, kLower><<<(ncols + 63) / 64, 64, 0, st>>>(nb, ncols, Tm, ldt, B, ldb);
+    constexpr int kCols = kTrsmWaves * kTrsmCols;
+    trsm_small_kernel<T, kLower><<<(ncols + kCols - 1) / kCols, 64 * kTrsmWaves, 0, st>>>(
+        nb, ncols, Tm, ldt, B, ldb);
     return hipGetLastError();
   }
   const int n1 = nb / 2, n2 = nb - n1;
@@ -296,28 +453,53 @@ hipError_t trsm(hipStream_t st, int nb, int ncols, const T *Tm, long ldt, T *B, 
   return trsm<T, false>(st, n1, ncols, T11, ldt, B1, ldb);
 }
 
-// leaf width for a block column of m rows: the widest power of two up to 32 whose
-// block fits the LDS (0: taller than the LDS holds even one column)
+// values a lane holds of a panel (half of its 256 VGPRs)
 template <typename T>
-int leaf_cols(int m) {
-  const long cap = static_cast<long>(kLeafLdsBytes / sizeof(T)) / std::max(m, 1);
+constexpr int panel_values() {
+  return static_cast<int>(512 / sizeof(T));
+}
+constexpr int kPanelMinCols = 4;
+// columns of a panel of m rows: the widest power of two up to 32 whose block is at most
+// 128 KiB, which the lanes hold; 0 (the steps in memory) where that is fewer than 4, past
+// 4096 FP64 or 2048 complex128 rows. (Wider panels, and a right-looking split into them,
+// were faster still but rounded every entry once per panel: FP64 n = 300 L U off by
+// 1.8e-15 ||A|| against 1.3e-15 for the halves below.)
+template <typename T>
+int panel_cols(int m) {
+  const long cap = static_cast<long>(131072 / sizeof(T)) / std::max(m, 1);
   int w = 0;
-  for (int c = 1; c <= kLeafMaxCols && c <= cap; c <<= 1) w = c;
-  return w;
+  for (int c = 1; c <= kPanelCols && c <= cap; c <<= 1) w = c;
+  return w >= kPanelMinCols ? w : 0;
+}
+
+template <typename T, int R>
+hipError_t launch_panel(hipStream_t st, int n, T *A, long lda, int k, int w, int *ipiv, int *info) {
+  if constexpr (R * kPanelMinCols > panel_values<T>()) {
+    return hipErrorInvalidValue;  // not reached: panel_cols gave 0
+  } else {
+    if (R * kPanelThreads < n - k) return launch_panel<T, 2 * R>(st, n, A, lda, k, w, ipiv, info);
+    constexpr int W = std::min(panel_values<T>() / R, kPanelCols);
+    if (w <= W / 2) panel_kernel<T, W / 2, R><<<1, kPanelThreads, 0, st>>>(n, A, lda, k, w, ipiv, info);
+    else panel_kernel<T, W, R><<<1, kPanelThreads, 0, st>>>(n, A, lda, k, w, ipiv, info);
+    return hipGetLastError();
+  }
 }
 
 template <typename T>
 hipError_t factor_block(hipStream_t st, int n, T *A, long lda, int k, int w, int *ipiv, int *info) {
   const int m = n - k;
-  const int lw = leaf_cols<T>(m);
-  if (w <= std::max(lw, lw == 0 ? 8 : 0)) {
-    if (lw > 0) leaf_lds_kernel<T><<<1, kLeafThreads, 0, st>>>(n, A, lda, k, w, ipiv, info);
-    else leaf_mem_kernel<T><<<1, kLeafThreads, 0, st>>>(n, A, lda, k, w, ipiv, info);
-    laswp_kernel<T><<<(n + 255) / 256, 256, 0, st>>>(n, A, lda, ipiv, k, k + w, k, k + w);
+  const int pw = panel_cols<T>(m);
+  hipError_t e;
+  if (w <= (pw == 0 ? 8 : pw)) {
+    if (pw > 0) {
+      if ((e = launch_panel<T, 1>(st, n, A, lda, k, w, ipiv, info)) != hipSuccess) return e;
+    } else {
+      leaf_mem_kernel<T><<<1, kLeafThreads, 0, st>>>(n, A, lda, k, w, ipiv, info);
+    }
+    laswp_kernel<T><<<(n + 255) / 256, 256, 0, st>>>(n, A, lda, ipiv, k, k + w, k, k + w, pw == 0);
     return hipGetLastError();
   }
   const int w1 = w / 2, w2 = w - w1;
-  hipError_t e;
   if ((e = factor_block<T>(st, n, A, lda, k, w1, ipiv, info)) != hipSuccess) return e;
   T *A11 = A + k + static_cast<long>(k) * lda;
   T *A12 = A + k + static_cast<long>(k + w1) * lda;
@@ -343,7 +525,7 @@ template <typename T>
 hipError_t launch_getrs(hipStream_t st, int n, int nrhs, const T *LU, long lda, const int *ipiv,
                         T *B, long ldb) {
   if (n <= 0 || nrhs <= 0) return hipSuccess;
-  laswp_kernel<T><<<(nrhs + 255) / 256, 256, 0, st>>>(nrhs, B, ldb, ipiv, 0, n, 0, 0);
+  laswp_kernel<T><<<(nrhs + 255) / 256, 256, 0, st>>>(nrhs, B, ldb, ipiv, 0, n, 0, 0, true);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if ((e = trsm<T, true>(st, n, nrhs, LU, lda, B, ldb)) != hipSuccess) return e;
