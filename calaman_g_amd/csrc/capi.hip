@@ -359,13 +359,14 @@ clm_status_t bank_powers(hipStream_t st, int n, const T *A, long lda, T *bank, l
 // Paterson-Stockmeyer on the device, the reference's structure
 // (src/paterson_stockmeyer/interface.cppm:364-419) with each B_j built inside
 // the epilogue of the Horner product that consumes it. The first `have` powers
-// (A^2 .. A^(have+1)) are already in the bank. x_scale multiplies every Horner
+// (A^2 .. A^(have+1)) are already in the bank; info (when given): two zeros. x_scale multiplies every Horner
 // product P X (2^-(b s) when A and its bank are unscaled and the 2^-s is folded
 // into the coefficients; exact, as every operand scaling here is a power of two).
 template <typename T>
 clm_status_t ps_evaluate(hipStream_t st, int n, const T *coef, int degree, const T *A, long lda,
                          T *P, long ldp, T *bank, long stride, T *scratch, long ld_scratch,
-                         int s_requested, int have = 0, double x_scale = 1.0) {
+                         int s_requested, int have = 0, double x_scale = 1.0,
+                         int *info = nullptr) {
   const clm_ps_plan p = ps_plan(degree, s_requested);
   CLM_TRY(bank_powers(st, n, A, lda, bank, stride, have + 2, p.num_powers + 1));
   const T *X = (p.r < 1) ? nullptr : (p.s >= 2) ? bank + static_cast<long>(p.s - 2) * stride : A;
@@ -378,7 +379,7 @@ clm_status_t ps_evaluate(hipStream_t st, int n, const T *coef, int degree, const
     return remaining < p.s ? remaining : p.s;
   };
   CLM_TRY_HIP(launch_build_block(st, n, buf[cur], ld[cur], coef + static_cast<long>(p.r) * p.s,
-                                 terms(p.r), A, lda, bank, stride, static_cast<long>(n)));
+                                 terms(p.r), A, lda, bank, stride, static_cast<long>(n), info));
   for (int j = p.r - 1; j >= 0; --j) {
     const int next = 1 - cur;
     GemmArgs<T> g;
@@ -802,33 +803,19 @@ ReadbackRing *ring_of(int device) {
   return &r;
 }
 
-// out[0 .. count-1] = the device values src[0 .. count-1] once the stream reaches
-// them. pinned = false takes a pageable copy and a stream synchronization and
-// allocates nothing.
-// `after` (when given) enqueues work that need not precede the values: it runs on the
-// device while the host waits for them.
-template <typename R, typename After = std::nullptr_t>
-clm_status_t read_back(hipStream_t st, int device, const R *src, int count, double *out,
-                       bool pinned, After after = nullptr) {
-  auto launch_after = [&]() -> hipError_t {
-    if constexpr (std::is_same_v<After, std::nullptr_t>) return hipSuccess;
-    else return after();
-  };
-  ReadbackRing *ring = pinned ? ring_of(device) : nullptr;
-  if (!ring) {
-    R host[kMaxNormPower] = {};
-    CLM_TRY_HIP(hipMemcpyAsync(host, src, sizeof(R) * count, hipMemcpyDeviceToHost, st));
-    CLM_TRY_HIP(launch_after());
-    CLM_TRY_HIP(hipStreamSynchronize(st));
-    for (int i = 0; i < count; ++i) out[i] = static_cast<double>(host[i]);
-    return CLM_STATUS_SUCCESS;
-  }
+// A slot of the device's ring for one hand-over: enqueue(vals, flag, seq) launches what
+// writes the values and then the flag; out[0 .. count-1] are read once the flag shows seq.
+// `after` enqueues work that need not precede the values: it runs on the device while
+// the host waits for them.
+template <typename Enqueue, typename After>
+clm_status_t hand_over(hipStream_t st, ReadbackRing *ring, int count, double *out, Enqueue enqueue,
+                       After after) {
   const unsigned ticket = ring->next.fetch_add(1, std::memory_order_relaxed);
   const unsigned seq = ticket + 1 == 0 ? 1 : ticket + 1;
   const int slot = static_cast<int>(ticket % kRingSlots);
   ReadbackSlot *h = ring->host + slot;
-  CLM_TRY_HIP(launch_publish(st, src, count, ring->dev[slot].vals, &ring->dev[slot].seq, seq));
-  CLM_TRY_HIP(launch_after());
+  CLM_TRY_HIP(enqueue(ring->dev[slot].vals, &ring->dev[slot].seq, seq));
+  CLM_TRY_HIP(after());
   const auto t0 = std::chrono::steady_clock::now();
   while (__atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) != seq) {
     if (std::chrono::steady_clock::now() - t0 > kSpinLimit) {
@@ -842,12 +829,54 @@ clm_status_t read_back(hipStream_t st, int device, const R *src, int count, doub
   return CLM_STATUS_SUCCESS;
 }
 
+// out[0 .. count-1] = the device values src[0 .. count-1] once the stream reaches
+// them. pinned = false takes a pageable copy and a stream synchronization and
+// allocates nothing.
+template <typename R, typename After>
+clm_status_t read_back(hipStream_t st, int device, const R *src, int count, double *out,
+                       bool pinned, After after) {
+  ReadbackRing *ring = pinned ? ring_of(device) : nullptr;
+  if (!ring) {
+    R host[kMaxNormPower] = {};
+    CLM_TRY_HIP(hipMemcpyAsync(host, src, sizeof(R) * count, hipMemcpyDeviceToHost, st));
+    CLM_TRY_HIP(after());
+    CLM_TRY_HIP(hipStreamSynchronize(st));
+    for (int i = 0; i < count; ++i) out[i] = static_cast<double>(host[i]);
+    return CLM_STATUS_SUCCESS;
+  }
+  return hand_over(
+      st, ring, count, out,
+      [&](double *vals, unsigned *flag, unsigned seq) {
+        return launch_publish(st, src, count, vals, flag, seq);
+      },
+      after);
+}
+
+// out[0 .. count-1] = the 1-norms of count n x n matrices mstride elements apart;
+// colsums: count * n values, dnorms: count values (both scratch)
+template <typename T, typename After>
+clm_status_t read_norms(hipStream_t st, int device, int n, const T *A, long lda, long mstride,
+                        int count, real_t<T> *colsums, real_t<T> *dnorms, double *out, bool pinned,
+                        After after) {
+  if (ReadbackRing *ring = pinned ? ring_of(device) : nullptr)
+    return hand_over(
+        st, ring, count, out,
+        [&](double *vals, unsigned *flag, unsigned seq) {
+          return launch_norm1_publish<T>(st, n, A, lda, mstride, count, colsums, vals, flag, seq);
+        },
+        after);
+  for (int i = 0; i < count; ++i)
+    CLM_TRY_HIP(launch_norm1<T>(st, n, A + i * mstride, lda, colsums, dnorms + i));
+  return read_back(st, device, dnorms, count, out, false, after);
+}
+
+constexpr auto kNothing = []() -> hipError_t { return hipSuccess; };
+
 template <typename T>
 clm_status_t read_norm1(hipStream_t st, int n, const T *A, long lda, real_t<T> *colsum,
                         real_t<T> *norm, int device = -1, bool pinned = false) {
-  CLM_TRY_HIP(launch_norm1(st, n, A, lda, colsum));
   double v = 0;
-  CLM_TRY(read_back(st, device, colsum, 1, &v, pinned));
+  CLM_TRY(read_norms<T>(st, device, n, A, lda, 0, 1, colsum, colsum, &v, pinned, kNothing));
   *norm = static_cast<real_t<T>>(v);
   return CLM_STATUS_SUCCESS;
 }
@@ -886,7 +915,6 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
   // their exponent arrays and find A's row and column exponents for the half format,
   // which A's first split then takes instead of a pass of its own (unused when the
   // plan picks the bfloat16 format)
-  CLM_TRY_HIP(launch_norm1(st, n, dA, lda, ws.colsum));
   double norm_v = 0;
   auto ahead = [&]() -> hipError_t {
     if (!use_split) return hipSuccess;
@@ -898,7 +926,8 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
     }
     return hipSuccess;
   };
-  CLM_TRY(read_back(st, c->device, ws.colsum, 1, &norm_v, may_allocate, ahead));
+  CLM_TRY(read_norms<T>(st, c->device, n, dA, lda, 0, 1, ws.colsum, ws.colsum, &norm_v,
+                        may_allocate, ahead));
   const real_t<T> norm = static_cast<real_t<T>>(norm_v);
   if (!std::isfinite(norm)) return CLM_STATUS_INVALID_VALUE;
 
@@ -944,15 +973,6 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
         CLM_TRY(bank_powers<T>(st, n, dA, lda, ws.bank, stride, formed + 1, q));
       }
       const int fresh = q - formed;  // powers A^(formed+1) .. A^q
-      if (n >= 4) {
-        CLM_TRY_HIP(launch_norm1_powers(st, n, ws.bank + static_cast<long>(formed - 1) * stride,
-                                        stride, fresh, reinterpret_cast<real_t<T> *>(ws.As),
-                                        dnorms + (formed - 1)));
-      } else {
-        for (int k = formed + 1; k <= q; ++k)
-          CLM_TRY_HIP(launch_norm1(st, n, ws.bank + static_cast<long>(k - 2) * stride, n,
-                                   ws.colsum, dnorms + (k - 2)));
-      }
       // behind this wait, the split variant splits A^q as a left operand when the plan
       // from the norms known so far has a block above q (the next power A^(q+1) is then
       // likely wanted and starts from those planes; otherwise they are replaced): the
@@ -970,8 +990,11 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
         }
         return hipSuccess;
       };
-      CLM_TRY(read_back(st, c->device, dnorms + (formed - 1), fresh, pn + formed, may_allocate,
-                        power_ahead));
+      // (below order 4 As is shorter than four columns of sums; one serves there)
+      real_t<T> *sums = n >= 4 ? reinterpret_cast<real_t<T> *>(ws.As) : ws.colsum;
+      CLM_TRY(read_norms<T>(st, c->device, n, ws.bank + static_cast<long>(formed - 1) * stride, n,
+                            stride, fresh, sums, dnorms + (formed - 1), pn + formed, may_allocate,
+                            power_ahead));
       formed = q;
       const bool more = use_split ? split_worth_next_power(pn, q, n, split, w_new)
                                   : worth_next_power(pn, q, is_single<T>());
@@ -1037,12 +1060,12 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
     } else {
       CLM_TRY(ps_evaluate<T>(st, n, pcoef, p.m, src, ld_src, target, ld_target, ws.bank,
                              static_cast<long>(ws.stride), other, ld_other, p.ps_block, q - 1,
-                             x_scale));
+                             x_scale, dInfo));
     }
   } else {
     CLM_TRY(ps_evaluate<T>(st, n, pcoef, p.m, src, ld_src, target, ld_target, ws.bank,
                            static_cast<long>(ws.stride), other, ld_other, p.ps_block, q - 1,
-                           x_scale));
+                           x_scale, dInfo));
   }
   if (plan) plan->fp8_gemms = p.fp8_gemms;
 
@@ -1070,7 +1093,8 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
     std::swap(cur, nxt);
     std::swap(ldc, ldn);
   }
-  if (dInfo) CLM_TRY_HIP(launch_fill_int(st, dInfo, 2, 0));
+  // (the plain form's polynomial has written it)
+  if (dInfo && use_split) CLM_TRY_HIP(launch_fill_int(st, dInfo, 2, 0));
   return CLM_STATUS_SUCCESS;
 }
 
@@ -1551,7 +1575,7 @@ template <typename R>
 clm_status_t read_device_values(hipStream_t st, int device, const R *src, int count, double *out) {
   if (src == nullptr || out == nullptr || count < 1 || count > kMaxNormPower)
     return CLM_STATUS_INVALID_VALUE;
-  return read_back(st, device, src, count, out, true);
+  return read_back(st, device, src, count, out, true, kNothing);
 }
 template clm_status_t read_device_values<double>(hipStream_t, int, const double *, int, double *);
 template clm_status_t read_device_values<float>(hipStream_t, int, const float *, int, double *);

@@ -221,12 +221,13 @@ hipError_t launch_gemm(hipStream_t stream, const GemmArgs<T> &g);
 template <typename T>
 hipError_t launch_norm1(hipStream_t stream, int n, const T *A, long lda, real_t<T> *colsum,
                         real_t<T> *out = nullptr);
-// the 1-norms of count n x n blocks (leading dimension n) `stride` elements apart:
-// column sums into colsums (count * n values), maxima into out[0 .. count-1];
-// each bit for bit launch_norm1's
+// the 1-norms of count n x n matrices mstride elements apart (leading dimension lda), each
+// bit for bit launch_norm1's, straight into host-mapped vals[0 .. count-1], then *flag =
+// seq; colsums: room for count * n sums
 template <typename T>
-hipError_t launch_norm1_powers(hipStream_t stream, int n, const T *bank, long stride, int count,
-                               real_t<T> *colsums, real_t<T> *out);
+hipError_t launch_norm1_publish(hipStream_t stream, int n, const T *A, long lda, long mstride,
+                                int count, real_t<T> *colsums, double *vals, unsigned *flag,
+                                unsigned seq);
 // bank[k-2] *= 2^(-k s) for k = 2 .. count + 1 (n x n blocks, leading dimension n)
 template <typename T>
 hipError_t launch_scale_powers(hipStream_t stream, int n, T *bank, long stride, int count, int s);
@@ -249,7 +250,7 @@ hipError_t launch_scale_copy(hipStream_t stream, int n, double f, const T *in, l
 // A(i,j) *= mul, m x n in place
 template <typename T>
 hipError_t launch_lascl(hipStream_t stream, size_t m, size_t n, double mul, T *A, size_t lda);
-// B = coef[0] I + coef[1] X1 + sum_t coef[t] bank[t-2]
+// B = coef[0] I + coef[1] X1 + sum_t coef[t] bank[t-2]; info[0], info[1] = 0 (when given)
 // launch_build_block for FP64 on the 64 x 64 element-wise tiling, with each row's
 // tagged exponent (generation gen, the half-format splits' encoding) into row_e
 hipError_t launch_build_block_rows(hipStream_t stream, int n, double *Bout, long ldb,
@@ -259,7 +260,7 @@ hipError_t launch_build_block_rows(hipStream_t stream, int n, double *Bout, long
 template <typename T>
 hipError_t launch_build_block(hipStream_t stream, int n, T *Bout, long ldb, const T *coef,
                               int nterms, const T *X1, long ldx1, const T *bank, long stride,
-                              long ldbank);
+                              long ldbank, int *info = nullptr);
 // P = (*alpha) I
 template <typename T>
 hipError_t launch_set_scaled_identity(hipStream_t stream, int n, T *P, long ldp, const T *alpha);

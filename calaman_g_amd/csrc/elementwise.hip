@@ -180,9 +180,10 @@ template <typename T>
 __global__ void __launch_bounds__(kEW)
     build_block_kernel(int n, T *__restrict__ Bout, long ldb, const T *__restrict__ coef,
                        int nterms, const T *__restrict__ X1, long ldx1, const T *__restrict__ bank,
-                       long stride, long ldbank) {
+                       long stride, long ldbank, int *info) {
   const int i = blockIdx.x * kEW + threadIdx.x;
   const long j = blockIdx.y;
+  if (info && i < 2 && j == 0) info[i] = 0;
   if (i >= n) return;
   T acc = (i == j) ? coef[0] : ops<T>::zero();
   if (nterms > 1) acc = ops<T>::mad(coef[1], X1[i + j * ldx1], acc);
@@ -218,6 +219,90 @@ __global__ void publish_kernel(const R *__restrict__ src, int count, double *val
   __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// The hand-over of norms in fewer launches than reduce, max, publish (each costs about
+// 4.5 us of the stream whatever it does; a call reads norms back two or three times).
+// vals[b] = the maximum of values + b * n (max_reduce_kernel's, NaN wins), b < count, then
+// the flag, as publish_kernel
+template <typename R>
+__global__ void __launch_bounds__(1024)
+    max_publish_kernel(int n, const R *__restrict__ values, int count, double *vals,
+                       unsigned *flag, unsigned seq) {
+  __shared__ R red[16];
+  const int tid = threadIdx.x;
+  for (int b = 0; b < count; ++b) {
+    const R *v = values + static_cast<long>(b) * n;
+    R best = 0;
+    for (int i = tid; i < n; i += 1024) {
+      const R x = v[i];
+      if (x > best || isnan(x)) best = x;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const R o = __shfl_xor(best, off);
+      if (o > best || isnan(o)) best = o;
+    }
+    if ((tid & 63) == 0) red[tid >> 6] = best;
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < 16; ++w)
+        if (red[w] > best || isnan(red[w])) best = red[w];
+      vals[b] = static_cast<double>(best);
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    __threadfence_system();
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// The same from the matrices themselves, for orders one workgroup reads at once: wave w
+// folds columns w, w + 16, ... in reduce_columns_kernel's order (virtual lane l + 64 q in
+// register q of lane l; its tree's first two levels add registers, the other six are
+// shuffles; a virtual lane past n holds +0, which changes no sum).
+template <typename T>
+__global__ void __launch_bounds__(1024)
+    norm1_publish_kernel(int n, const T *__restrict__ A, long lda, long mstride, int count,
+                         double *vals, unsigned *flag, unsigned seq) {
+  using R = real_t<T>;
+  __shared__ R red[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int b = 0; b < count; ++b) {
+    const T *X = A + static_cast<long>(b) * mstride;
+    R best = 0;
+    for (int j = wave; j < n; j += 16) {
+      R v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int t = lane + 64 * q;
+        v[q] = t < n ? modulus(X[t + static_cast<long>(j) * lda]) : R(0);
+      }
+      v[0] = v[0] + v[2];
+      v[1] = v[1] + v[3];
+      v[0] = v[0] + v[1];
+#pragma unroll
+      for (int s = 32; s > 0; s >>= 1) {
+        const R o = __shfl_down(v[0], s, 64);
+        if (lane < s) v[0] = v[0] + o;
+      }
+      const R cs = __shfl(v[0], 0, 64);
+      if (cs > best || isnan(cs)) best = cs;
+    }
+    if (lane == 0) red[wave] = best;
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < 16; ++w)
+        if (red[w] > best || isnan(red[w])) best = red[w];
+      vals[b] = static_cast<double>(best);
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    __threadfence_system();
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 __global__ void fill_int_kernel(int *d, int count, int v) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < count) d[i] = v;
@@ -240,14 +325,23 @@ hipError_t launch_norm1(hipStream_t stream, int n, const T *A, long lda, real_t<
   return hipGetLastError();
 }
 
+// One workgroup to order 128 (128 KiB of FP64: about the time of a launch to read); above
+// that the columns' sums need the chip, and the maximum and the hand-over share a launch.
 template <typename T>
-hipError_t launch_norm1_powers(hipStream_t stream, int n, const T *bank, long stride, int count,
-                               real_t<T> *colsums, real_t<T> *out) {
-  if (n < 1 || count < 1) return hipSuccess;
-  hipLaunchKernelGGL((reduce_columns_kernel<T, 0, 0>), dim3(n, count), dim3(kRB), 0, stream, bank,
-                     colsums, static_cast<size_t>(n), static_cast<size_t>(n), stride);
-  hipLaunchKernelGGL(max_reduce_kernel<real_t<T>>, dim3(count), dim3(kRB), 0, stream, n, colsums,
-                     out);
+hipError_t launch_norm1_publish(hipStream_t stream, int n, const T *A, long lda, long mstride,
+                                int count, real_t<T> *colsums, double *vals, unsigned *flag,
+                                unsigned seq) {
+  constexpr int kOneWorkgroup = 128;
+  static_assert(kOneWorkgroup <= kRB, "a lane's four registers hold a column");
+  if (n <= kOneWorkgroup) {
+    hipLaunchKernelGGL(norm1_publish_kernel<T>, dim3(1), dim3(1024), 0, stream, n, A, lda, mstride,
+                       count, vals, flag, seq);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((reduce_columns_kernel<T, 0, 0>), dim3(n, count), dim3(kRB), 0, stream, A,
+                     colsums, static_cast<size_t>(n), static_cast<size_t>(lda), mstride);
+  hipLaunchKernelGGL(max_publish_kernel<real_t<T>>, dim3(1), dim3(1024), 0, stream, n, colsums,
+                     count, vals, flag, seq);
   return hipGetLastError();
 }
 
@@ -327,10 +421,10 @@ hipError_t launch_lascl(hipStream_t stream, size_t m, size_t n, double mul, T *A
 template <typename T>
 hipError_t launch_build_block(hipStream_t stream, int n, T *Bout, long ldb, const T *coef,
                               int nterms, const T *X1, long ldx1, const T *bank, long stride,
-                              long ldbank) {
+                              long ldbank, int *info) {
   if (n < 1 || nterms < 1) return hipSuccess;
   hipLaunchKernelGGL(build_block_kernel<T>, col_grid(n, n), dim3(kEW), 0, stream, n, Bout, ldb,
-                     coef, nterms, X1, ldx1, bank, stride, ldbank);
+                     coef, nterms, X1, ldx1, bank, stride, ldbank, info);
   return hipGetLastError();
 }
 
@@ -368,16 +462,16 @@ hipError_t launch_fill_int(hipStream_t stream, int *d, int count, int v) {
 
 #define CLM_INSTANTIATE(T)                                                                         \
   template hipError_t launch_norm1<T>(hipStream_t, int, const T *, long, real_t<T> *, real_t<T> *); \
+  template hipError_t launch_norm1_publish<T>(hipStream_t, int, const T *, long, long, int,        \
+                                              real_t<T> *, double *, unsigned *, unsigned);        \
   template hipError_t launch_scale_coef<T>(hipStream_t, const T *, T *, int, int, int);            \
   template hipError_t launch_scale_powers<T>(hipStream_t, int, T *, long, int, int);               \
-  template hipError_t launch_norm1_powers<T>(hipStream_t, int, const T *, long, int, real_t<T> *,  \
-                                             real_t<T> *);                                         \
   template hipError_t launch_lange<T>(hipStream_t, int, size_t, size_t, const T *, size_t,          \
                                       real_t<T> *, real_t<T> *);                                   \
   template hipError_t launch_scale_copy<T>(hipStream_t, int, double, const T *, long, T *, long);  \
   template hipError_t launch_lascl<T>(hipStream_t, size_t, size_t, double, T *, size_t);           \
   template hipError_t launch_build_block<T>(hipStream_t, int, T *, long, const T *, int, const T *, \
-                                            long, const T *, long, long);                          \
+                                            long, const T *, long, long, int *);                   \
   template hipError_t launch_set_scaled_identity<T>(hipStream_t, int, T *, long, const T *);       \
   template hipError_t launch_copy<T>(hipStream_t, int, const T *, long, T *, long);
 
