@@ -158,6 +158,10 @@ constexpr int threads_of(int cfg) { return cfg == CLM_BATCH_TILE_128W16 ? 1024 :
 template <typename T, int CFG>
 constexpr size_t lds_bytes() {
   constexpr int c = effective_cfg<T>(CFG);
+  // complex FP64 asked for a tile above 64 x 64 runs the 64 x 64 one with a CU to itself:
+  // the LDS it claims leaves no room for a second workgroup of any product tile above 32
+  if constexpr (std::is_same_v<T, zd> && CFG != c && CFG != CLM_BATCH_TILE_128W16)
+    return 140 * 1024;
   if constexpr (c == CLM_BATCH_TILE_128W16) {
     if constexpr (is_cplx<T>()) return cplx_lds<T, 128, 128, 1024>();
     else return real_lds<T, 128, 128, 32, 1024>();
@@ -190,6 +194,7 @@ __device__ __forceinline__ double uniform(double v) {
 // A size or lane index the compiler cannot look through: what a pass derives from it is
 // computed in the pass instead of being carried across the whole chain in registers.
 __device__ __forceinline__ int opaque_s(int v) {
+  v = uniform(v);  // every caller's size is uniform; unoptimized builds need to be told
   asm volatile("" : "+s"(v));
   return v;
 }
@@ -977,13 +982,15 @@ __global__ void __launch_bounds__(threads_of(CFG))
 // the exit once the counter passes `count`.
 // waves per SIMD the registers are held to: a workgroup's barriers and loads hide behind
 // the other workgroups of its CU (1024 complex64 of order 144 on the 32 x 32 tile: 2.25 ms
-// at 3 waves, 1.93 at 4, 2.2 at 5, where the plan's FP64 constants spill in the loop)
+// at 3 waves, 1.93 at 4, 2.2 at 5, where the plan's FP64 constants spill in the loop). Real
+// FP32 stops at 3: held to 4 it spills 20 B a lane (856 matrices of order 9 to 85: 501 us at
+// 3 waves, 527 at 4)
 template <typename T, int CFG>
 constexpr int min_waves() {
   if (threads_of(CFG) == 1024) return 4;
-  if (CFG == CLM_BATCH_TILE_32) return std::is_same_v<T, zd> ? 3 : 4;
+  if (CFG == CLM_BATCH_TILE_32) return std::is_same_v<T, zc> || std::is_same_v<T, double> ? 4 : 3;
   if (CFG == CLM_BATCH_TILE_64)
-    return std::is_same_v<T, float> ? 4 : std::is_same_v<T, zd> ? 2 : 3;
+    return std::is_same_v<T, zd> ? 2 : 3;
   return 1;
 }
 
@@ -1048,10 +1055,14 @@ bool g_tune_init = false;
 // complex]; the last bucket also serves every larger order. Measured over whole mixed
 // batches (orders 16 to 256): a table of few tiles keeps the groups few and their tails
 // short, so it beats the per-bucket winners by up to a quarter (2048 complex64: 12.1 ms
-// against 16.1 ms; 2048 FP64: 6.5 against 7.8). Adjoint plans: the per-bucket winners.
+// against 16.1 ms; 2048 FP64: 6.5 against 7.8). complex FP64 above order 96 keeps a CU to
+// itself (tile 2, see lds_bytes): two workgroups a CU finish smaller orders sooner (1500 of
+// 16 to 160: 7.0 ms against 8.5) but stretch the longest
+// chains, which end the launch (1000 of 16 to 256: 17.7 against 16.8; 512 of them next to 512
+// FP64: 18.2 against 13.2). Adjoint plans: the per-bucket winners.
 constexpr int kDefaultTiles[2][2][2][kBuckets] = {
     {{{0, 1, 1, 1, 1, 1, 4, 4}, {0, 0, 0, 1, 1, 1, 4, 4}},
-     {{0, 1, 1, 1, 1, 1, 1, 1}, {0, 0, 0, 1, 0, 1, 1, 4}}},
+     {{0, 1, 1, 1, 1, 1, 1, 1}, {0, 0, 0, 2, 2, 2, 2, 2}}},
     {{{0, 1, 3, 3, 1, 2, 4, 4}, {0, 1, 0, 2, 1, 1, 4, 4}},
      {{0, 1, 2, 2, 1, 1, 4, 4}, {0, 1, 0, 1, 0, 1, 1, 1}}}};
 
