@@ -428,8 +428,8 @@ __global__ void set_info_kernel(int *info, int v) {
 // ---- the Taylor route -------------------------------------------------------------------
 constexpr double kTaylorMaxNorm1 = 32.0;
 
-// a value that is not less than best, NaN included, wins
-__device__ inline double nan_max_(double best, double v) { return v <= best ? best : v; }
+// the larger; a NaN on either side stays
+__device__ inline double nan_max_(double best, double v) { return v > best || isnan(v) ? v : best; }
 
 // stats[j] = column j's 1-norm, stats[n + j] = its part off the diagonal
 template <typename W>

@@ -32,6 +32,10 @@ def _spectrum(n, cplx, kind, norm, seed):
 
 
 def _run(a, uplo, dev, nbytes=None):
+    return _call(a, uplo, dev, nbytes)[0]
+
+
+def _call(a, uplo, dev, nbytes=None, want_info=0):
     n, ld = a.shape[0], a.shape[0] + 1
     dt = torch.complex128 if np.iscomplexobj(a) else torch.float64
     buf = np.full((n, ld), np.nan, dtype=a.dtype)
@@ -44,10 +48,10 @@ def _run(a, uplo, dev, nbytes=None):
     work = torch.empty(size, dtype=torch.uint8, device=dev)
     info = torch.full((1,), -3, dtype=torch.int32, device=dev)
     assert cg.expm_herm_cm(uplo, n, da, ld, de, ld, work, info) == 0
-    assert int(info.item()) == 0
+    assert want_info is None or int(info.item()) == want_info
     out = de.cpu().numpy()
     assert np.all(out[:, n:] == 7.0)
-    return out[:, :n].T
+    return out[:, :n].T, int(info.item())
 
 
 def _jacobi_bytes(n, size):
@@ -78,3 +82,19 @@ def test_a_workspace_of_the_sweeps_size_still_serves(dev, cplx):
     ref = oh.expm_herm(a)
     err = np.linalg.norm(_run(a, "U", dev, nbytes) - ref) / np.linalg.norm(ref)
     assert err <= 1e-12
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("n,i,j", [(2, 0, 0), (2, 1, 1), (2, 0, 1), (64, 0, 0), (64, 31, 31),
+                                   (64, 5, 40), (512, 0, 0), (512, 255, 255), (512, 511, 511),
+                                   (512, 3, 300)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_a_value_that_is_not_finite_goes_to_the_sweeps(dev, cplx, n, i, j, bad):
+    """wherever it stands: the same status, info and result as in the sweeps' workspace"""
+    a = _spectrum(n, cplx, "full", 4.0, n)
+    a[i, j] = a[j, i] = bad
+    print(f"expm_herm n={n} cplx={cplx} a[{i},{j}]={bad}", flush=True)
+    want, want_info = _call(a, "U", dev, _jacobi_bytes(n, 16 if cplx else 8), None)
+    got, info = _call(a, "U", dev, None, None)
+    assert info == want_info
+    np.testing.assert_array_equal(got, want)  # NaN where it has NaN
