@@ -852,8 +852,15 @@ clm_status_t read_back(hipStream_t st, int device, const R *src, int count, doub
       after);
 }
 
+// the order from which an n x n block holds the column sums of the up to kMaxNormPower - 1
+// powers read back together
+constexpr int kSumsTogetherN = 4;
+static_assert(kMaxNormPower - 1 <= kSumsTogetherN, "a block holds the sums");
+
 // out[0 .. count-1] = the 1-norms of count n x n matrices mstride elements apart;
-// colsums: count * n values, dnorms: count values (both scratch)
+// colsums: count * n values (n below order kSumsTogetherN), dnorms: count values (both
+// scratch). Without the ring one pair of launches serves all of them (a pair a matrix put
+// 5 us on every clm_expm_noalloc_d call: n = 8, ||A||_1 = 1, 82 -> 86 us).
 template <typename T, typename After>
 clm_status_t read_norms(hipStream_t st, int device, int n, const T *A, long lda, long mstride,
                         int count, real_t<T> *colsums, real_t<T> *dnorms, double *out, bool pinned,
@@ -865,8 +872,11 @@ clm_status_t read_norms(hipStream_t st, int device, int n, const T *A, long lda,
           return launch_norm1_publish<T>(st, n, A, lda, mstride, count, colsums, vals, flag, seq);
         },
         after);
-  for (int i = 0; i < count; ++i)
-    CLM_TRY_HIP(launch_norm1<T>(st, n, A + i * mstride, lda, colsums, dnorms + i));
+  if (n >= kSumsTogetherN)
+    CLM_TRY_HIP(launch_norm1<T>(st, n, A, lda, colsums, dnorms, mstride, count));
+  else
+    for (int i = 0; i < count; ++i)
+      CLM_TRY_HIP(launch_norm1<T>(st, n, A + i * mstride, lda, colsums, dnorms + i));
   return read_back(st, device, dnorms, count, out, false, after);
 }
 
@@ -954,8 +964,9 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
     const long stride = static_cast<long>(ws.stride);
     bool pca_is_a = false, ca_split = false, ca_fp8 = false;
     const double w_new = p0.ps_split == CLM_SPLIT_BF16X6 ? 0.35 : 0.2;
-    // the power norms land in the first bytes of S and their column sums in As
-    // (both unused until the polynomial; As holds q - 1 <= 4 columns of sums for n >= 4)
+    // the powers' column sums go to As (unused until the polynomial) and, without the
+    // ring, their norms to the first bytes of S; the last launch of the ring's form writes
+    // the norms to the host
     real_t<T> *dnorms = reinterpret_cast<real_t<T> *>(ws.S);
     int formed = 1;  // A^1 .. A^formed exist
     for (;;) {
@@ -990,8 +1001,7 @@ clm_status_t expm_impl(clm_ctx *ctx, hipStream_t st, int n, const T *dA, int lda
         }
         return hipSuccess;
       };
-      // (below order 4 As is shorter than four columns of sums; one serves there)
-      real_t<T> *sums = n >= 4 ? reinterpret_cast<real_t<T> *>(ws.As) : ws.colsum;
+      real_t<T> *sums = n >= kSumsTogetherN ? reinterpret_cast<real_t<T> *>(ws.As) : ws.colsum;
       CLM_TRY(read_norms<T>(st, c->device, n, ws.bank + static_cast<long>(formed - 1) * stride, n,
                             stride, fresh, sums, dnorms + (formed - 1), pn + formed, may_allocate,
                             power_ahead));

@@ -217,10 +217,11 @@ template <typename T>
 hipError_t launch_gemm(hipStream_t stream, const GemmArgs<T> &g);
 
 // ---- element-wise and reduction kernels ------------------------------------------------
-// 1-norm in two launches (colsums, NaN-propagating max into dColsum[0]).
+// 1-norm in two launches (colsums, NaN-propagating max into colsum[0], or out[0] when
+// given); of count > 1 matrices mstride elements apart: count * n sums, out[0 .. count-1]
 template <typename T>
 hipError_t launch_norm1(hipStream_t stream, int n, const T *A, long lda, real_t<T> *colsum,
-                        real_t<T> *out = nullptr);
+                        real_t<T> *out = nullptr, long mstride = 0, int count = 1);
 // the 1-norms of count n x n matrices mstride elements apart (leading dimension lda), each
 // bit for bit launch_norm1's, straight into host-mapped vals[0 .. count-1], then *flag =
 // seq; colsums: room for count * n sums

@@ -316,11 +316,11 @@ inline dim3 col_grid(size_t rows, size_t cols) {
 
 template <typename T>
 hipError_t launch_norm1(hipStream_t stream, int n, const T *A, long lda, real_t<T> *colsum,
-                        real_t<T> *out) {
-  if (n < 1) return hipSuccess;
-  hipLaunchKernelGGL((reduce_columns_kernel<T, 0, 0>), dim3(n), dim3(kRB), 0, stream, A, colsum,
-                     static_cast<size_t>(n), static_cast<size_t>(lda));
-  hipLaunchKernelGGL(max_reduce_kernel<real_t<T>>, dim3(1), dim3(kRB), 0, stream, n, colsum,
+                        real_t<T> *out, long mstride, int count) {
+  if (n < 1 || count < 1) return hipSuccess;
+  hipLaunchKernelGGL((reduce_columns_kernel<T, 0, 0>), dim3(n, count), dim3(kRB), 0, stream, A,
+                     colsum, static_cast<size_t>(n), static_cast<size_t>(lda), mstride);
+  hipLaunchKernelGGL(max_reduce_kernel<real_t<T>>, dim3(count), dim3(kRB), 0, stream, n, colsum,
                      out ? out : colsum);
   return hipGetLastError();
 }
@@ -461,7 +461,8 @@ hipError_t launch_fill_int(hipStream_t stream, int *d, int count, int v) {
 }
 
 #define CLM_INSTANTIATE(T)                                                                         \
-  template hipError_t launch_norm1<T>(hipStream_t, int, const T *, long, real_t<T> *, real_t<T> *); \
+  template hipError_t launch_norm1<T>(hipStream_t, int, const T *, long, real_t<T> *, real_t<T> *,  \
+                                      long, int);                                                  \
   template hipError_t launch_norm1_publish<T>(hipStream_t, int, const T *, long, long, int,        \
                                               real_t<T> *, double *, unsigned *, unsigned);        \
   template hipError_t launch_scale_coef<T>(hipStream_t, const T *, T *, int, int, int);            \
