@@ -186,19 +186,21 @@ hipError_t launch_large(hipStream_t stream, const GemmArgs<T> &g) {
     // 16 waves of 32 x 16 over slices of 16: 1044 -> 997 us at n = 2048 against 8 waves
     // of 32 x 32 (twice the waves over the same LDS)
     return launch_piped<T, 128, 64, 16, 32, 16, 1>(stream, g);
-  } else if constexpr (std::is_same_v<T, double>) {
-    // whole tiles and slices at 16-byte aligned columns: no bounds anywhere and 16-byte
-    // column pieces out of LDS, 280 against 285 us at n = 2048
-    const bool fast = g.M % 128 == 0 && g.N % 128 == 0 && g.K % 32 == 0 && g.lda % 2 == 0 &&
-                      g.ldb % 2 == 0 && aligned16(g.A) && aligned16(g.B);
-    if (fast) {
-      const int tiles_m = g.M / 128, tiles_n = g.N / 128;
-      hipLaunchKernelGGL((rgemm_mfma<double, 128, 128, 32, 32, 1024, 32>),
-                         dim3(tiles_m * tiles_n), dim3(1024), 0, stream, g, tiles_m, tiles_n);
-      return hipGetLastError();
-    }
-    return launch_piped<T, 128, 128, 32, 32, 32, 1>(stream, g);
   } else {
+    if constexpr (!std::is_same_v<T, zc>) {
+      // real, whole tiles and slices at 16-byte aligned columns: no bounds anywhere and
+      // 16-byte column pieces out of LDS, at n = 2048 FP64 280 against 285 us, at n = 4096
+      // FP32 1063 against 1097 us, FP32 8192 x 8192 x 64 116 against 122 us
+      constexpr int EV = 16 / sizeof(T);
+      const bool fast = g.M % 128 == 0 && g.N % 128 == 0 && g.K % 32 == 0 && g.lda % EV == 0 &&
+                        g.ldb % EV == 0 && aligned16(g.A) && aligned16(g.B);
+      if (fast) {
+        const int tiles_m = g.M / 128, tiles_n = g.N / 128;
+        hipLaunchKernelGGL((rgemm_mfma<T, 128, 128, 32, 32, 1024, 32>), dim3(tiles_m * tiles_n),
+                           dim3(1024), 0, stream, g, tiles_m, tiles_n);
+        return hipGetLastError();
+      }
+    }
     return launch_piped<T, 128, 128, 32, 32, 32, 1>(stream, g);
   }
 }
