@@ -131,7 +131,7 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 constexpr int kCus = 256;
 
 // The workgroup tile of a product: 32 x 32 (4 waves of one MFMA tile), 64 x 64 (16 such
-// waves) or the large tile (16 waves of 2 x 2 or 2 x 1 MFMA tiles). All three run the
+// waves, or 4 of 2 x 2) or the large tile (16 waves of 2 x 2 or 2 x 1 MFMA tiles). All three run the
 // same k order, so the choice is speed only: the estimate is the rounds of tiles the
 // 256 CUs take, times the measured time of one tile and k (ns, beyond the launch).
 // A lone 32 x 32 tile per CU has one wave per SIMD and waits on its loads (`one`).
@@ -174,9 +174,11 @@ constexpr TileCost kLarge<zc>{128, 128, 268.0, 268.0};
 template <>
 constexpr TileCost kLarge<zd>{128, 64, 243.0, 243.0};
 
+inline long tiles_of(const TileCost &t, int m, int n) {
+  return static_cast<long>((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+}
 inline double estimate(const TileCost &t, int m, int n) {
-  const long tiles = static_cast<long>((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-  const long rounds = (tiles + kCus - 1) / kCus;
+  const long rounds = (tiles_of(t, m, n) + kCus - 1) / kCus;
   return rounds == 1 ? t.one : static_cast<double>(rounds) * t.more;
 }
 
@@ -213,6 +215,13 @@ hipError_t launch_product(hipStream_t stream, const GemmArgs<T> &g) {
   if (l <= m && l <= s) return launch_large<T>(stream, g);
   if (m <= s) {
     constexpr int BK = std::is_same_v<T, float> ? 64 : 32;  // a vector a lane and slice
+    if constexpr (std::is_same_v<T, float>) {
+      // FP32 past two tiles a CU: 4 waves of 2 x 2 MFMA tiles, eight workgroups a CU, which
+      // need no whole rounds (n = 1664 102 -> 98 us, 1728 107 -> 101, 1650 104 -> 98); up to
+      // two, twice the waves of a tile hide more (n = 1024 25 us against 33)
+      if (tiles_of(kMedium<T>, g.M, g.N) > 2 * kCus)
+        return launch_piped<T, 64, 64, 16, 32, 32, 1>(stream, g);
+    }
     return launch_piped<T, 64, 64, BK, 16, 16, 1>(stream, g);
   }
   return launch_piped<T, 32, 32, 32, 16, 16, 2>(stream, g);

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [  # small, medium and large tiles; one below, at and above an edge; k down to 1
     (1, 1, 1), (3, 2, 5), (31, 33, 32), (32, 32, 31), (33, 31, 33), (64, 65, 63), (95, 97, 1),
-    (257, 33, 130), (33, 511, 70), (999, 1001, 67), (1024, 1000, 64), (1921, 1930, 47),
+    (257, 33, 130), (33, 511, 70), (999, 1001, 67), (1024, 1000, 64), (1664, 1664, 48),
+    (1650, 1687, 37), (1700, 1601, 1), (1921, 1930, 47),
     (2047, 2049, 33), (2048, 2048, 31)]
 
 
