@@ -63,6 +63,7 @@ constexpr int kBuckets = CLM_BATCH_BUCKETS;
 constexpr int kMaxBatchN = 4096;
 constexpr int kTiles = CLM_BATCH_TILES;
 constexpr int kGroups = 4 * kTiles;  // (element type, tile) pairs
+constexpr int kXcds = 8;
 constexpr size_t kHeadBytes = 256;  // the groups' queue counters at the head of the workspace
 
 template <typename T>
@@ -1074,6 +1075,14 @@ void tune_defaults() {
   g_tune_init = true;
 }
 
+int compute_units(int device) {
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+      cus < 1)
+    cus = 256;
+  return cus;
+}
+
 int bucket_of(int n) {
   const int b = (n - 1) / 32;
   return b < kBuckets ? b : kBuckets - 1;
@@ -1110,34 +1119,73 @@ int group_of(int dtype, int cfg) {
   return t * kTiles + cfg;
 }
 
+// complex FP64 above the 32 x 32 tile: chains that slow each other most on one CU
+bool is_wide(int group) {
+  return group >= group_of(CLM_DTYPE_C128, 0) && group % kTiles != CLM_BATCH_TILE_32;
+}
+
+// How many workgroups a CU may hold, per group (0: as many as fit). The groups of a plan are
+// launched side by side and the device packs each one's workgroups by itself: since a CU's
+// registers hold three chains and more (two at most before, one of complex FP64 above the
+// 32 x 32 tile), a batch of one or two matrices a CU had come to put three on some, whose
+// slowed chains end the launch. So while there is room every matrix has its CU; then two
+// share one, the wide ones still none while there is room; from 2.25 matrices a CU on the
+// device is better left to fill up, except with the shortest chains of all. us, before that
+// change / with it / as claimed here: 400 FP64 of order 4 to 40 373 / 462 / 374, 500 FP32
+// 236 / 295 / 238, 200 FP64 371 / 371 / 312; left to fill up, 600 FP64 of order 33 to 64
+// 664 / 511, held to two 650; held to two, 700 FP64 of order 2 to 12 361 / 419 / 368.
+enum Spread { kAlone, kHalves, kFull };
+Spread spread_groups(const int *group_count, int count, int nmax, int cus, int *per_cu) {
+  constexpr int kTiny = 16;
+  // workgroups go round the XCDs, every group from the first one: what an XCD gets at most
+  int wide = 0, other = 0;
+  for (int g = 0; g < kGroups; ++g)
+    (is_wide(g) ? wide : other) += (group_count[g] + kXcds - 1) / kXcds;
+  const int room = cus / kXcds;
+  const Spread how = wide + other <= room             ? kAlone
+                     : wide + (other + 1) / 2 <= room ? kHalves
+                                                      : kFull;
+  const bool two = 4 * count <= 9 * cus || (nmax <= kTiny && count <= 4 * cus);
+  for (int g = 0; g < kGroups; ++g)
+    per_cu[g] = how == kAlone || (how == kHalves && is_wide(g)) ? 1 : how == kHalves || two ? 2 : 0;
+  return how;
+}
+
 // workgroups resident at once on the device for one kernel instantiation
 template <typename T, int CFG>
 int resident_workgroups(int device) {
   static int cached[64] = {};
   int &r = cached[device & 63];
   if (r == 0) {
-    int blocks = 0, cus = 0;
+    int blocks = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, expm_batched_kernel<T, CFG>, threads_of(CFG), 0) !=
             hipSuccess ||
         blocks < 1)
       blocks = 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-        cus < 1)
-      cus = 256;
-    r = blocks * cus;
+    r = blocks * compute_units(device);
   }
   return r;
 }
 
+// LDS a workgroup claims beyond its own `used` bytes to share its CU with one other claimant
+// (per_cu 2) or with none (1); 0: no claim. Why: spread_groups.
+inline size_t lds_claim(int per_cu, size_t used) {
+  constexpr size_t kOfTwo = 56 * 1024, kAlone = 112 * 1024;
+  static_assert(2 * kOfTwo <= 160 * 1024 && 3 * kOfTwo > 160 * 1024 && kAlone + kOfTwo > 160 * 1024,
+                "of a CU's 160 KiB");
+  const size_t want = per_cu == 1 ? kAlone : per_cu == 2 ? kOfTwo : 0;
+  return want > used ? want - used : 0;
+}
+
 template <typename T, int CFG>
 hipError_t launch_group(hipStream_t st, int device, const BatchDesc *desc, int count, int *queue,
-                        char *work, clm_batch_result *results) {
+                        char *work, clm_batch_result *results, int per_cu) {
   const T *coef = inv_factorials<T>(device);
   if (!coef) return hipErrorInvalidValue;
   const int grid = std::min(count, resident_workgroups<T, CFG>(device));
-  hipLaunchKernelGGL((expm_batched_kernel<T, CFG>), dim3(grid), dim3(threads_of(CFG)), 0, st, desc,
-                     count,
-                     queue, work, results, coef);
+  hipLaunchKernelGGL((expm_batched_kernel<T, CFG>), dim3(grid), dim3(threads_of(CFG)),
+                     lds_claim(per_cu, lds_bytes<T, CFG>()), st, desc, count, queue, work, results,
+                     coef);
   return hipGetLastError();
 }
 
@@ -1172,15 +1220,12 @@ hipError_t launch_adjoint_group(hipStream_t st, int device, const BatchDesc *des
   static int cached[64] = {};
   int &resident = cached[device & 63];
   if (resident == 0) {
-    int blocks = 0, cus = 0;
+    int blocks = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, expm_adjoint_kernel<T, CFG>, threads_of(CFG), 0) !=
             hipSuccess ||
         blocks < 1)
       blocks = 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-        cus < 1)
-      cus = 256;
-    resident = blocks * cus;
+    resident = blocks * compute_units(device);
   }
   hipLaunchKernelGGL((expm_adjoint_kernel<T, CFG>), dim3(std::min(count, resident)),
                      dim3(threads_of(CFG)), 0,
@@ -1207,18 +1252,18 @@ hipError_t launch_adjoint_type(int cfg, hipStream_t st, int device, const BatchD
 
 template <typename T>
 hipError_t launch_type(int cfg, hipStream_t st, int device, const BatchDesc *desc, int count,
-                       int *queue, char *work, clm_batch_result *results) {
+                       int *queue, char *work, clm_batch_result *results, int per_cu) {
   switch (cfg) {
   case CLM_BATCH_TILE_32:
-    return launch_group<T, CLM_BATCH_TILE_32>(st, device, desc, count, queue, work, results);
+    return launch_group<T, CLM_BATCH_TILE_32>(st, device, desc, count, queue, work, results, per_cu);
   case CLM_BATCH_TILE_64:
-    return launch_group<T, CLM_BATCH_TILE_64>(st, device, desc, count, queue, work, results);
+    return launch_group<T, CLM_BATCH_TILE_64>(st, device, desc, count, queue, work, results, per_cu);
   case CLM_BATCH_TILE_128x64:
-    return launch_group<T, CLM_BATCH_TILE_128x64>(st, device, desc, count, queue, work, results);
+    return launch_group<T, CLM_BATCH_TILE_128x64>(st, device, desc, count, queue, work, results, per_cu);
   case CLM_BATCH_TILE_128:
-    return launch_group<T, CLM_BATCH_TILE_128>(st, device, desc, count, queue, work, results);
+    return launch_group<T, CLM_BATCH_TILE_128>(st, device, desc, count, queue, work, results, per_cu);
   default:
-    return launch_group<T, CLM_BATCH_TILE_128W16>(st, device, desc, count, queue, work, results);
+    return launch_group<T, CLM_BATCH_TILE_128W16>(st, device, desc, count, queue, work, results, per_cu);
   }
 }
 
@@ -1231,10 +1276,12 @@ struct clm_batch_plan {
   int count = 0;
   int group_count[clm::kGroups] = {};  // matrices per (element type, tile) group
   int group_start[clm::kGroups] = {};
-  double group_cost[clm::kGroups] = {};  // sum of n^3 (x4 complex, x2 FP64) of the members
+  // n^3 (x4 complex, x2 FP64) of the members: the sum, or the largest with a CU for each
+  double group_cost[clm::kGroups] = {};
   int launch_order[clm::kGroups] = {};   // non-empty groups, costliest first
   int launch_lane[clm::kGroups] = {};    // 0: the caller's stream, i > 0: side[i - 1]
   int num_launch = 0;
+  int per_cu[clm::kGroups] = {};  // workgroups a CU may hold (lds_claim), 0: as many as fit
   clm::BatchDesc *d_desc = nullptr;    // grouped, each group in decreasing cost
   bool ad = false;                     // records the adjoint tape; backward allowed
   int ckpt = 0;
@@ -1308,6 +1355,7 @@ clm_status_t build_plan(int count, const clm_batch_entry *entries, const int *fo
   if (ad && (ckpt < 1 || ckpt > 64)) return CLM_STATUS_INVALID_VALUE;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return CLM_STATUS_NOT_INITIALIZED;
+  const int cus = compute_units(dev);
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     if (!g_tune_init) tune_defaults();
@@ -1318,14 +1366,16 @@ clm_status_t build_plan(int count, const clm_batch_entry *entries, const int *fo
     const double n = entries[i].n;
     return n * n * n * (is_complex_code(entries[i].dtype) ? 4.0 : 1.0);
   };
+  int nmax = 0;
+  for (int i = 0; i < count; ++i) nmax = std::max(nmax, entries[i].n);
   std::vector<int> cfg(count);
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     for (int i = 0; i < count; ++i) {
       const clm_batch_entry &e = entries[i];
+      const int p = precision_of(e.dtype), c = is_complex_code(e.dtype);
       cfg[i] = forced_cfg ? *forced_cfg
-                          : g_tune[ad ? 1 : 0][precision_of(e.dtype)][is_complex_code(e.dtype)]
-                                  [bucket_of(e.n)];
+                          : g_tune[ad ? 1 : 0][p][c][bucket_of(e.n)];
     }
   }
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
@@ -1337,6 +1387,7 @@ clm_status_t build_plan(int count, const clm_batch_entry *entries, const int *fo
   plan->device = dev;
   plan->count = count;
   plan->host_desc.resize(count);
+  double longest[kGroups] = {};
   size_t off = kHeadBytes;
   for (int k = 0; k < count; ++k) {
     const int i = order[k];
@@ -1367,10 +1418,15 @@ clm_status_t build_plan(int count, const clm_batch_entry *entries, const int *fo
       d.tape_off = static_cast<long long>(off);
       off += Layout::align(tape_bytes_of(e.dtype, e.n, ckpt));
     }
-    plan->group_count[group_of(e.dtype, cfg[i])] += 1;
-    plan->group_cost[group_of(e.dtype, cfg[i])] +=
-        cost(i) * ((e.dtype == CLM_DTYPE_F64 || e.dtype == CLM_DTYPE_C128) ? 2.0 : 1.0);
+    const int g = group_of(e.dtype, cfg[i]);
+    plan->group_count[g] += 1;
+    const double c = cost(i) * (precision_of(e.dtype) ? 2.0 : 1.0);
+    plan->group_cost[g] += c;
+    longest[g] = std::max(longest[g], c);
   }
+  // a group whose matrices all have their CU takes as long as its longest chain
+  if (spread_groups(plan->group_count, count, nmax, cus, plan->per_cu) == kAlone)
+    std::copy(longest, longest + kGroups, plan->group_cost);
   for (int g = 1; g < kGroups; ++g)
     plan->group_start[g] = plan->group_start[g - 1] + plan->group_count[g - 1];
   // Longest-processing-time lanes: the groups in decreasing cost, each on the
@@ -1438,10 +1494,14 @@ clm_status_t launch_plan(clm_ctx *ctx, hipStream_t st, const clm_batch_plan *pla
     const BatchDesc *desc = plan->d_desc + plan->group_start[g];
     const int cfg = g % kTiles;
     switch (g / kTiles) {
-    case 0: return launch_type<float>(cfg, s, plan->device, desc, count, queue + g, base, results);
-    case 1: return launch_type<double>(cfg, s, plan->device, desc, count, queue + g, base, results);
-    case 2: return launch_type<zc>(cfg, s, plan->device, desc, count, queue + g, base, results);
-    default: return launch_type<zd>(cfg, s, plan->device, desc, count, queue + g, base, results);
+    case 0: return launch_type<float>(cfg, s, plan->device, desc, count, queue + g, base, results,
+                                  plan->per_cu[g]);
+    case 1: return launch_type<double>(cfg, s, plan->device, desc, count, queue + g, base, results,
+                                  plan->per_cu[g]);
+    case 2: return launch_type<zc>(cfg, s, plan->device, desc, count, queue + g, base, results,
+                                  plan->per_cu[g]);
+    default: return launch_type<zd>(cfg, s, plan->device, desc, count, queue + g, base, results,
+                                  plan->per_cu[g]);
     }
   });
 }

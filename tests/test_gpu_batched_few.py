@@ -1,0 +1,50 @@
+"""GPU: batches around one and two matrices a CU, where a plan's tiles and the workgroups a
+CU may hold change (256 CUs: 256 and 512 matrices, 576 above which the device fills up),
+and tiny orders, which are held to two up to four a CU -- of one element type and of
+several. Every member is bit for bit clm_expm_*'s result on the same input.
+"""
+import numpy as np
+import pytest
+import torch
+
+import calaman_g_amd as cg
+from calaman_g_amd.expm import BatchPlan, expm_cm
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [torch.float32, torch.float64, torch.complex64, torch.complex128]
+
+
+def _inputs(dtype, orders, dev):
+    """per order: the matrix (column-major) and its exponential by the single call"""
+    out = {}
+    for n in orders:
+        gen = torch.Generator(device="cuda").manual_seed(n)
+        a = torch.randn((n, n), generator=gen, device=dev, dtype=dtype)
+        a = a * (3.0 / float(a.abs().sum(1).max()))
+        e = torch.empty_like(a)
+        work = torch.empty(cg.expm_buffer_size(n, dtype), dtype=torch.uint8, device=dev)
+        assert expm_cm(n, a, n, e, n, work)[0] == 0
+        out[n] = (a, e)
+    return out
+
+
+@pytest.mark.parametrize("types", [[t] for t in TYPES] + [TYPES[:1] + TYPES[2:3], TYPES],
+                         ids=["f32", "f64", "c64", "c128", "f32+c64", "all"])
+@pytest.mark.parametrize("count,lo,hi", [(1, 33, 33), (40, 100, 210), (255, 2, 40), (256, 33, 64),
+                                         (257, 20, 70), (300, 40, 44), (512, 2, 40), (513, 33, 64),
+                                         (577, 2, 50), (900, 2, 12)])
+def test_members_are_the_single_results(dev, types, count, lo, hi):
+    rng = np.random.default_rng(count)
+    orders = sorted(set(rng.integers(lo, hi + 1, size=9).tolist()))
+    known = {t: _inputs(t, orders, dev) for t in types}
+    picks = [(types[int(rng.integers(len(types)))], int(rng.choice(orders))) for _ in range(count)]
+    entries = [(n, known[t][n][0], n, torch.empty_like(known[t][n][0]), n) for t, n in picks]
+    print(f"batch of {count}, orders {lo}..{hi}, {len(types)} types", flush=True)
+    plan = BatchPlan(entries)
+    work, res = plan.workspace(), plan.results_buffer()
+    assert plan.launch(work, res) == 0
+    assert all(r["status"] == 0 for r in BatchPlan.decode_results(res))
+    for (t, n), (_, _, _, e, _) in zip(picks, entries):
+        want = known[t][n][1]
+        assert torch.equal(e.view(torch.uint8), want.view(torch.uint8)), (t, n)
