@@ -1067,6 +1067,16 @@ constexpr int kDefaultTiles[2][2][2][kBuckets] = {
     {{{0, 1, 3, 3, 1, 2, 4, 4}, {0, 1, 0, 2, 1, 1, 4, 4}},
      {{0, 1, 2, 2, 1, 1, 4, 4}, {0, 1, 0, 1, 0, 1, 1, 1}}}};
 
+// The same for forward plans of few matrices (few_matrices): the longest chain alone is the launch's time, so a matrix takes the tile of the quickest
+// chain whatever that does to a full CU. us, the tiles before per-bucket defaults / default
+// table / this one: 4 FP32 of order 128 408 / 433 / 339, 4 FP64 of order 224 2123 / 2247 /
+// 1512, 64 complex64 of order 48 183 / 201 / 181, 300 of them 239 / 260 / 237, 64 complex128
+// of order 64 389 / 426 / 387. Only while the (type, tile) groups are no more than the
+// streams they run on, or they queue behind each other: 64 of four types, order 4 to 40,
+// 462 us with the default table's 6 groups, 770 with 8.
+constexpr int kFewTiles[2][2][kBuckets] = {{{0, 1, 3, 3, 1, 1, 4, 4}, {0, 1, 0, 1, 1, 1, 4, 4}},
+                                           {{0, 1, 2, 2, 1, 1, 4, 4}, {0, 1, 0, 1, 0, 1, 4, 4}}};
+
 void tune_defaults() {
   for (int a = 0; a < 2; ++a)
     for (int p = 0; p < 2; ++p)
@@ -1119,6 +1129,13 @@ int group_of(int dtype, int cfg) {
   return t * kTiles + cfg;
 }
 
+// kFewTiles' tile of an entry, or the tuning table's above order 256 (the caller holds its
+// mutex)
+int few_tile(const clm_batch_entry &e) {
+  const int p = precision_of(e.dtype), c = is_complex_code(e.dtype);
+  return (e.n <= 32 * kBuckets ? kFewTiles : g_tune[0])[p][c][bucket_of(e.n)];
+}
+
 // complex FP64 above the 32 x 32 tile: chains that slow each other most on one CU
 bool is_wide(int group) {
   return group >= group_of(CLM_DTYPE_C128, 0) && group % kTiles != CLM_BATCH_TILE_32;
@@ -1149,6 +1166,37 @@ Spread spread_groups(const int *group_count, int count, int nmax, int cus, int *
   for (int g = 0; g < kGroups; ++g)
     per_cu[g] = how == kAlone || (how == kHalves && is_wide(g)) ? 1 : how == kHalves || two ? 2 : 0;
   return how;
+}
+
+// whether kFewTiles serve a forward plan: a CU for every matrix, or half a one in a single
+// group or beside wide chains; no more groups than lanes; and tuning tables that nobody has
+// changed (the caller holds their mutex)
+bool few_matrices(int count, const clm_batch_entry *entries, int cus, int lanes) {
+  if (count > 2 * cus) return false;
+  int used[kGroups] = {}, per_cu[kGroups], nmax = 0;
+  bool all_c64 = true;
+  for (int i = 0; i < count; ++i) {
+    const clm_batch_entry &e = entries[i];
+    nmax = std::max(nmax, e.n);
+    all_c64 &= e.dtype == CLM_DTYPE_C64;
+    const int p = precision_of(e.dtype), c = is_complex_code(e.dtype);
+    if (!std::equal(g_tune[0][p][c], g_tune[0][p][c] + kBuckets, kDefaultTiles[0][p][c]))
+      return false;
+    ++used[group_of(e.dtype, few_tile(e))];
+  }
+  int groups = 0;
+  bool wide = false;
+  for (int g = 0; g < kGroups; ++g) {
+    groups += used[g] > 0;
+    wide |= used[g] > 0 && is_wide(g);
+  }
+  const Spread how = spread_groups(used, count, 0, cus, per_cu);
+  // (complex64 whose largest order is 41 to 64: at half a CU each too, 300 of order 16 to 64
+  // 241 / 262 / 229 us; below, one group of the 32 x 32 tile is as quick, above, the larger
+  // orders' default tiles are)
+  const bool c64_to_64 = all_c64 && nmax > 40 && nmax <= 64;
+  return groups <= lanes &&
+         (how == kAlone || (how == kHalves && (groups == 1 || wide || c64_to_64)));
 }
 
 // workgroups resident at once on the device for one kernel instantiation
@@ -1371,10 +1419,13 @@ clm_status_t build_plan(int count, const clm_batch_entry *entries, const int *fo
   std::vector<int> cfg(count);
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
+    const bool few =
+        !forced_cfg && !ad && few_matrices(count, entries, cus, 1 + clm_batch_plan::kSide);
     for (int i = 0; i < count; ++i) {
       const clm_batch_entry &e = entries[i];
       const int p = precision_of(e.dtype), c = is_complex_code(e.dtype);
       cfg[i] = forced_cfg ? *forced_cfg
+               : few      ? few_tile(e)
                           : g_tune[ad ? 1 : 0][p][c][bucket_of(e.n)];
     }
   }
