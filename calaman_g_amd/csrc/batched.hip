@@ -157,12 +157,8 @@ constexpr int effective_cfg(int cfg) {
 constexpr int threads_of(int cfg) { return cfg == CLM_BATCH_TILE_128W16 ? 1024 : 256; }
 
 template <typename T, int CFG>
-constexpr size_t lds_bytes() {
+constexpr size_t tile_lds() {
   constexpr int c = effective_cfg<T>(CFG);
-  // complex FP64 asked for a tile above 64 x 64 runs the 64 x 64 one with a CU to itself:
-  // the LDS it claims leaves no room for a second workgroup of any product tile above 32
-  if constexpr (std::is_same_v<T, zd> && CFG != c && CFG != CLM_BATCH_TILE_128W16)
-    return 140 * 1024;
   if constexpr (c == CLM_BATCH_TILE_128W16) {
     if constexpr (is_cplx<T>()) return cplx_lds<T, 128, 128, 1024>();
     else return real_lds<T, 128, 128, 32, 1024>();
@@ -176,6 +172,16 @@ constexpr size_t lds_bytes() {
     else if constexpr (c == CLM_BATCH_TILE_128x64) return real_lds<T, 128, 64, kBK>();
     else return real_lds<T, 128, 128, kBK>();
   }
+}
+
+// LDS of the forward chain. Complex FP64 asked for a tile above 64 x 64 runs the 64 x 64 one
+// with a CU to itself: what it claims leaves no room for a second workgroup of any product
+// tile above 32.
+template <typename T, int CFG>
+constexpr size_t lds_bytes() {
+  if constexpr (std::is_same_v<T, zd> && CFG != effective_cfg<T>(CFG) && CFG != CLM_BATCH_TILE_128W16)
+    return 140 * 1024;
+  else return tile_lds<T, CFG>();
 }
 
 // A value every lane of the wave holds, re-declared uniform: the compiler then
@@ -565,7 +571,9 @@ __device__ void wg_fill(int n, T *dst, long ld, T v) {
 // the adjoint kernel's LDS: the product's stages, at least one transpose tile
 template <typename T, int CFG>
 constexpr size_t kAdjointLds() {
-  return lds_bytes<T, CFG>() > transpose_lds<T>() ? lds_bytes<T, CFG>() : transpose_lds<T>();
+  // not the forward's claim: two backward sweeps share a CU (300 complex128 of order 100 on
+  // tile 2, forward and backward, 5.1 ms with a CU each, 4.4 ms)
+  return tile_lds<T, CFG>() > transpose_lds<T>() ? tile_lds<T, CFG>() : transpose_lds<T>();
 }
 
 // the adjoint tape of one matrix (layout above tape_blocks)
