@@ -1759,14 +1759,9 @@ clm_status_t autotune(clm_ctx *ctx, hipStream_t st, int path, int dtype, int nma
   CLM_TRY(get_tuning(path, dtype, chosen));
   const bool single = precision_of(dtype) == 0;
   const bool cplx = is_complex_code(dtype);
-  // candidate tiles: those that are distinct for this type (128 x 128 of 4 waves
-  // exists for real FP32 only, 128 x 64 for all but complex FP64)
-  auto distinct = [&](int cfg) {
-    if (cfg == CLM_BATCH_TILE_128W16) return true;
-    if (cfg == CLM_BATCH_TILE_128) return single && !cplx;
-    if (cfg == CLM_BATCH_TILE_128x64) return single || !cplx;
-    return true;
-  };
+  // candidate tiles: those that are distinct for this type (128 x 128 of 4 waves exists for
+  // real FP32 only; 128 x 64 is, for complex FP64, 64 x 64 with a CU to itself)
+  auto distinct = [&](int cfg) { return cfg != CLM_BATCH_TILE_128 || (single && !cplx); };
   const bool adj = path == 1;
   for (int b = 0; b < kBuckets && 32 * b < nmax; ++b) {
     const int n = std::min(32 * b + 16, nmax);

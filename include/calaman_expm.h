@@ -456,8 +456,8 @@ typedef struct clm_batch_plan clm_batch_plan;
 #define CLM_BATCH_BUCKETS 8
 #define CLM_BATCH_TILE_32 0     /* 32 x 32 */
 #define CLM_BATCH_TILE_64 1     /* 64 x 64 */
-#define CLM_BATCH_TILE_128x64 2 /* 128 x 64 (complex FP64: 64 x 64) */
-#define CLM_BATCH_TILE_128 3    /* 128 x 128 of 4 waves (real FP32 only; others: their largest) */
+#define CLM_BATCH_TILE_128x64 2 /* 128 x 64 (complex FP64: 64 x 64, one workgroup a CU) */
+#define CLM_BATCH_TILE_128 3    /* 128 x 128 of 4 waves (real FP32 only; others: as tile 2) */
 #define CLM_BATCH_TILE_128W16 4 /* 128 x 128 of 16 waves (every type) */
 #define CLM_BATCH_TILES 5
 
@@ -487,7 +487,11 @@ clm_status_t clm_expm_batched_graph(clm_ctx *ctx, clm_stream_t stream, clm_batch
  * of the bucket's middle order under every tile and keeps the fastest. ms_out
  * (optional, CLM_BATCH_TILES * CLM_BATCH_BUCKETS floats) receives
  * ms[bucket * CLM_BATCH_TILES + tile] (0 for a tile that is not distinct for the type).
- * Plans created afterwards use the new table. */
+ * Plans created afterwards use the new table. Its batches are of one order each: for
+ * many orders together the default table, which was measured on such batches, can be
+ * the faster one (4096 of orders 16 to 256, FP32 and complex64: 15.4 ms, tuned 16.0).
+ * While a type's table is the default one, forward plans of few matrices (about one
+ * a CU) take tiles chosen for the longest chain instead. */
 clm_status_t clm_expm_batched_get_tuning(int dtype, int *cfg);
 clm_status_t clm_expm_batched_set_tuning(int dtype, const int *cfg);
 clm_status_t clm_expm_batched_autotune(clm_ctx *ctx, clm_stream_t stream, int dtype, int nmax,

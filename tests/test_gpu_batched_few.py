@@ -48,3 +48,15 @@ def test_members_are_the_single_results(dev, types, count, lo, hi):
     for (t, n), (_, _, _, e, _) in zip(picks, entries):
         want = known[t][n][1]
         assert torch.equal(e.view(torch.uint8), want.view(torch.uint8)), (t, n)
+
+
+def test_the_tuner_times_complex128_with_a_cu_to_itself(dev):
+    """tile 2 is a launch of its own for complex128 (one workgroup a CU), tile 3 is not"""
+    saved = cg.batched_tuning(torch.complex128)
+    try:
+        table, ms = cg.batched_autotune(torch.complex128, nmax=40)
+        for b in (0, 1):
+            assert all(ms[b][t] > 0 for t in (0, 1, 2, 4)) and ms[b][3] == 0
+            assert ms[b][table[b]] == min(t for t in ms[b] if t > 0)
+    finally:
+        cg.set_batched_tuning(torch.complex128, saved)
