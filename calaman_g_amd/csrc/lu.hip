@@ -200,7 +200,7 @@ __device__ inline void group_argmax(long long &key, int &idx) {
   }
   unsigned long long has = __ballot(key == m);
   if constexpr (width < 64) has &= (1ull << width) - 1;  // the keys repeat past the group
-  if (m == -2) has = 0;  // no row in the group
+  if (__ballot(m != -2) == 0) has = 0;  // no row in the group
   int first = INT_MAX;
   while (has) {
     first = min(first, __builtin_amdgcn_readlane(idx, __ffsll(has) - 1));
@@ -278,9 +278,9 @@ __global__ void __launch_bounds__(kPanelThreads)
       if (!nonzero) atomicMin(info, row0 + j + 1);
     }
     __syncthreads();
-    // lane c of every wave takes column c of the two rows; a column's value then goes to
+    // lane c of every wave takes column c of the pivot row; a column's value then goes to
     // all lanes through a scalar register
-    const T prow = rows[set][0][lane % W], jrow = rows[set][1][lane % W];
+    const T prow = rows[set][0][lane % W];
     if (tid < w - j) blk[j + static_cast<long>(j + tid) * lda] = prow;
     const T pv = from_lane(prow, 0);
     const bool safe = cabs1(pv) >= min_normal<T>();
@@ -288,9 +288,9 @@ __global__ void __launch_bounds__(kPanelThreads)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = tid + kPanelThreads * r;
-      if (i == p && p != j) {
+      if (i == p && p != j) {  // one lane: its own reads, no other lane's registers
 #pragma unroll
-        for (int c = 0; c < W; ++c) a[r][c] = from_lane(jrow, c);
+        for (int c = 0; c < W; ++c) a[r][c] = rows[set][1][c];
       }
       T l = a[r][0];
       if (nonzero) l = safe ? ops<T>::mul(l, rp) : cdiv(l, pv);

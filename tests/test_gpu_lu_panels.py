@@ -51,6 +51,42 @@ def test_panels_reconstruct(dev, dt, n):
     assert np.all(np.abs(lo @ up - pa) <= 2 * (n + 4) * u * (np.abs(lo) @ np.abs(up)))
 
 
+@pytest.mark.parametrize("dt,n", [(torch.float64, 4096), (torch.float64, 4097), (torch.complex64, 4097),
+                                  (torch.complex128, 2048), (torch.complex128, 2050),
+                                  (torch.float32, 4097), (torch.float32, 8193)])
+def test_tall_panels_reconstruct(dev, dt, n):
+    """the tallest panels in registers (4 columns) and the first that run in memory, the same
+    bound; the products in 64 bits on the device"""
+    print(f"getrf n={n} {dt}", flush=True)
+    a = torch.from_numpy(_matrix(n, dt, n)).to(dev)
+    lu = a.t().contiguous()
+    ipiv = torch.zeros(n, dtype=torch.int32, device=dev)
+    info = torch.full((1,), -1, dtype=torch.int32, device=dev)
+    assert cg.getrf_cm(n, lu, n, ipiv, info) == 0 and int(info.item()) == 0
+    wide = torch.complex128 if dt.is_complex else torch.float64
+    lu = lu.t().to(wide)
+    perm = np.arange(n)
+    for k, q in enumerate(ipiv.cpu().numpy()):
+        perm[[k, q - 1]] = perm[[q - 1, k]]
+    lo, up = torch.tril(lu, -1) + torch.eye(n, dtype=wide, device=dev), torch.triu(lu)
+    err = (lo @ up - a.to(wide)[torch.from_numpy(perm).to(dev)]).abs()
+    u = np.finfo(NP[dt]).eps / 2
+    assert bool(torch.all(err <= 2 * (n + 4) * u * (lo.abs() @ up.abs())))
+
+
+@pytest.mark.parametrize("dt", list(NP))
+@pytest.mark.parametrize("rows", [(70, 200, 515), (3, 515), (511, 512), (600, 1112), (64, 63)])
+def test_equal_pivots_in_several_waves_take_the_first_row(dev, dt, rows):
+    """the largest entry of column 0 in several waves, in two rows of one lane (512 apart)
+    and on both sides of a wave's edge"""
+    n = 1300
+    a = _matrix(n, dt, 9)
+    a[:, 0] /= 2 * np.abs(a[:, 0]).max()
+    a[list(rows), 0] = 3.0
+    _, ipiv, info = _getrf(a, dt, dev)
+    assert info == 0 and int(ipiv[0]) == min(rows) + 1
+
+
 def test_equal_pivots_take_the_first_row(dev):
     n = 40
     a = np.ones((n, n))
