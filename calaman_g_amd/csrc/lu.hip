@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(kPanelThreads)
   }
 }
 
-// the same steps on the matrix in memory, for blocks taller than the LDS holds
+// the same steps on the matrix in memory, for blocks taller than the lanes hold
 template <typename T>
 __global__ void __launch_bounds__(kLeafThreads)
     leaf_mem_kernel(int n, T *A, long lda, int row0, int w, int *ipiv, int *info) {
@@ -453,32 +453,30 @@ hipError_t trsm(hipStream_t st, int nb, int ncols, const T *Tm, long ldt, T *B, 
   return trsm<T, false>(st, n1, ncols, T11, ldt, B1, ldb);
 }
 
-// values a lane holds of a panel (half of its 256 VGPRs)
-template <typename T>
-constexpr int panel_values() {
-  return static_cast<int>(512 / sizeof(T));
-}
 constexpr int kPanelMinCols = 4;
 // columns of a panel of m rows: the widest power of two up to 32 whose block is at most
-// 128 KiB, which the lanes hold; 0 (the steps in memory) where that is fewer than 4, past
-// 4096 FP64 or 2048 complex128 rows. (Wider panels, and a right-looking split into them,
-// were faster still but rounded every entry once per panel: FP64 n = 300 L U off by
-// 1.8e-15 ||A|| against 1.3e-15 for the halves below.)
+// 128 KiB, which the lanes hold (half of their 256 VGPRs); 0 (the steps in memory) where
+// that is fewer than 4, past 4096 FP64, 2048 complex128 or 8192 FP32 rows. (Wider panels,
+// and a right-looking split into them, were faster still but rounded every entry once per
+// panel: FP64 n = 300 L U off by 1.8e-15 ||A|| against 1.3e-15 for the halves below.)
+// In memory up to 8 columns make a panel, where one or two held in LDS did: FP64 n = 16000
+// 399 -> 376 ms, complex128 n = 8000 224 -> 148, complex64 n = 9000 180 -> 143.
 template <typename T>
-int panel_cols(int m) {
-  const long cap = static_cast<long>(131072 / sizeof(T)) / std::max(m, 1);
+constexpr int panel_cols(int m) {
+  const long cap = static_cast<long>(131072 / sizeof(T)) / (m < 1 ? 1 : m);
   int w = 0;
   for (int c = 1; c <= kPanelCols && c <= cap; c <<= 1) w = c;
   return w >= kPanelMinCols ? w : 0;
 }
 
+// w columns at R rows a lane, the fewest that reach row n
 template <typename T, int R>
 hipError_t launch_panel(hipStream_t st, int n, T *A, long lda, int k, int w, int *ipiv, int *info) {
-  if constexpr (R * kPanelMinCols > panel_values<T>()) {
+  constexpr int W = panel_cols<T>(kPanelThreads * (R / 2) + 1);  // at the fewest rows R serves
+  if constexpr (W == 0) {
     return hipErrorInvalidValue;  // not reached: panel_cols gave 0
   } else {
     if (R * kPanelThreads < n - k) return launch_panel<T, 2 * R>(st, n, A, lda, k, w, ipiv, info);
-    constexpr int W = std::min(panel_values<T>() / R, kPanelCols);
     if (w <= W / 2) panel_kernel<T, W / 2, R><<<1, kPanelThreads, 0, st>>>(n, A, lda, k, w, ipiv, info);
     else panel_kernel<T, W, R><<<1, kPanelThreads, 0, st>>>(n, A, lda, k, w, ipiv, info);
     return hipGetLastError();

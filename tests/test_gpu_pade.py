@@ -6,7 +6,7 @@ expm against an oracle, the singular and ill-scaled cases).
 
 * getrf: the pivots are the oracle's (and scipy's) exactly; L and U agree to 1e-13 of
   ||A||; P L U reconstructs A; a zero column reports its index in info; block
-  columns taller than the LDS holds (the in-memory leaf) at n = 8300 complex128.
+  columns taller than the registers hold (the panel in memory) at n = 8300 complex128.
 * getrs: the solve against numpy.linalg.solve.
 * pade: every degree against orc_pade (1e-13 FP64; FP32 within its precision).
 * expm_pade: the plan equals the oracle's (the same 1-norm, bit for bit for real input),
@@ -125,8 +125,8 @@ def test_getrf_zero_pivot_reports_column(dev):
 
 
 def test_getrf_tall_block_columns_in_memory(dev):
-    """n = 8300 complex128: the first block columns hold more rows than the LDS leaf
-    (8192 complex128 entries a column), so they run the in-memory leaf"""
+    """n = 8300 complex128: the first block columns hold more rows than the lanes hold
+    (2048 complex128 entries a column), so they run the panel in memory"""
     n = 8300
     torch.manual_seed(0)
     a = torch.randn((n, n), dtype=torch.complex128, device=dev)
