@@ -1589,6 +1589,7 @@ clm_status_t read_device_values(hipStream_t st, int device, const R *src, int co
 }
 template clm_status_t read_device_values<double>(hipStream_t, int, const double *, int, double *);
 template clm_status_t read_device_values<float>(hipStream_t, int, const float *, int, double *);
+template clm_status_t read_device_values<int>(hipStream_t, int, const int *, int, double *);
 
 }  // namespace clm
 

@@ -453,6 +453,8 @@ template hipError_t launch_publish<double>(hipStream_t, const double *, int, dou
                                            unsigned);
 template hipError_t launch_publish<float>(hipStream_t, const float *, int, double *, unsigned *,
                                           unsigned);
+template hipError_t launch_publish<int>(hipStream_t, const int *, int, double *, unsigned *,
+                                        unsigned);
 
 hipError_t launch_fill_int(hipStream_t stream, int *d, int count, int v) {
   if (count < 1) return hipSuccess;

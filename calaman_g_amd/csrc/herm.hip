@@ -115,10 +115,11 @@ __device__ inline void pair_of(int r, int t, int np2, int &p, int &q) {
 }
 
 // H = the uplo triangle of A mirrored (real diagonal), zero-padded to np x np, in the
-// working type W
+// working type W; V (when given) = I
 template <typename T, typename W>
 __global__ void __launch_bounds__(kThreads)
-    mirror_kernel(int n, int np, int upper, const T *__restrict__ A, long lda, W *__restrict__ H) {
+    mirror_kernel(int n, int np, int upper, const T *__restrict__ A, long lda, W *__restrict__ H,
+                  W *__restrict__ V) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
   const int j = blockIdx.y;
   if (i >= np) return;
@@ -129,6 +130,7 @@ __global__ void __launch_bounds__(kThreads)
     else v = widen(conj_(A[j + static_cast<long>(i) * lda]));
   }
   H[i + static_cast<long>(j) * np] = v;
+  if (V) V[i + static_cast<long>(j) * np] = ops<W>::from_real(i == j ? 1.0 : 0.0);
 }
 // E = the n x n result rounded to the caller's type
 template <typename T, typename W>
@@ -137,13 +139,6 @@ __global__ void __launch_bounds__(kThreads)
   const int i = blockIdx.x * kThreads + threadIdx.x;
   const int j = blockIdx.y;
   if (i < n) E[i + static_cast<long>(j) * lde] = narrow<T>(X[i + static_cast<long>(j) * n]);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kThreads) identity_kernel(int np, T *V) {
-  const int i = blockIdx.x * kThreads + threadIdx.x;
-  const int j = blockIdx.y;
-  if (i < np) V[i + static_cast<long>(j) * np] = ops<T>::from_real(i == j ? 1.0 : 0.0);
 }
 
 // colsq[j] = sum_i |H(i, j)|^2
@@ -179,8 +174,8 @@ __global__ void __launch_bounds__(kThreads)
   if (threadIdx.x == 0) *delta = u * sqrt(red[0]) / static_cast<R>(np);
 }
 
-__global__ void clear_count_kernel(unsigned *c) {
-  if (threadIdx.x == 0) *c = 0u;
+__global__ void clear_count_kernel(int *c) {
+  if (threadIdx.x == 0) *c = 0;
 }
 
 // local index l of a 64-wide pair (p, q) -> global index
@@ -198,7 +193,7 @@ __device__ inline int glob(int l, int p, int q) { return l < kB ? p * kB + l : q
 template <typename W>
 __global__ void __launch_bounds__(kSolveThreads)
     solve_kernel(int np, W *H, const real_t<W> *delta, int round, W *Qbuf, int *flags,
-                 unsigned *count) {
+                 int *count) {
   using R = real_t<W>;
   __shared__ W S[kP][kLd];
   __shared__ W Q[kP][kLd];
@@ -289,7 +284,7 @@ __global__ void __launch_bounds__(kSolveThreads)
   }
   if (threadIdx.x == 0) {
     flags[t] = any ? 1 : 0;
-    if (any) atomicAdd(count, 1u);
+    if (any) atomicAdd(count, 1);
   }
 }
 
@@ -548,7 +543,7 @@ clm_status_t herm_taylor(clm_ctx *ctx, int device, hipStream_t st, int upper, in
   HermTaylorWs<T> ws;
   ws.carve(work, n);
   const dim3 grid((n + kThreads - 1) / kThreads, n);
-  mirror_kernel<T, W><<<grid, kThreads, 0, st>>>(n, n, upper, A, lda, ws.H);
+  mirror_kernel<T, W><<<grid, kThreads, 0, st>>>(n, n, upper, A, lda, ws.H, nullptr);
   column_stats_kernel<W><<<n, kThreads, 0, st>>>(n, ws.H, ws.stats);
   fold_stats_kernel<W><<<1, kThreads, 0, st>>>(n, ws.H, ws.stats, ws.out);
   CLM_TRY_HIP(hipGetLastError());
@@ -578,8 +573,7 @@ clm_status_t herm_taylor(clm_ctx *ctx, int device, hipStream_t st, int upper, in
 template <typename T>
 struct HermWs {
   T *H = nullptr, *V = nullptr, *W = nullptr, *Q = nullptr;
-  int *flags = nullptr;
-  unsigned *count = nullptr;
+  int *flags = nullptr, *count = nullptr;
   real_t<T> *delta = nullptr, *colsq = nullptr;
   size_t carve(void *base, int n) {
     const size_t np = static_cast<size_t>((n + kP - 1) / kP) * kP;
@@ -590,7 +584,7 @@ struct HermWs {
     W = L.take<T>(np * np);
     Q = L.take<T>(k * kP * kP);
     flags = L.take<int>(k);
-    count = L.take<unsigned>(1);
+    count = L.take<int>(1);
     delta = L.take<real_t<T>>(1);
     colsq = L.take<real_t<T>>(np);
     return L.total();
@@ -630,8 +624,7 @@ clm_status_t expm_herm_impl(clm_ctx *ctx, hipStream_t st, int uplo, int n, const
   const int np2 = np / kB, k = np2 / 2;
   const dim3 grid_sq((np + kThreads - 1) / kThreads, np);
   mirror_kernel<T, W><<<grid_sq, kThreads, 0, st>>>(n, np, uplo == CLM_FILL_MODE_UPPER, A, lda,
-                                                    ws.H);
-  identity_kernel<W><<<grid_sq, kThreads, 0, st>>>(np, ws.V);
+                                                    ws.H, ws.V);
   colsq_kernel<W><<<np, kThreads, 0, st>>>(np, ws.H, ws.colsq);
   // the unit roundoff of the working precision, 2^-53
   delta_kernel<W><<<1, kThreads, 0, st>>>(np, ws.colsq, R(1.1102230246251565e-16), ws.delta);
@@ -645,9 +638,8 @@ clm_status_t expm_herm_impl(clm_ctx *ctx, hipStream_t st, int uplo, int n, const
       update_kernel<W><<<jobs, kThreads, 0, st>>>(np, ws.H, ws.V, r, ws.Q, ws.flags);
     }
     CLM_TRY_HIP(hipGetLastError());
-    unsigned rotated = 0;
-    CLM_TRY_HIP(hipMemcpyAsync(&rotated, ws.count, sizeof(unsigned), hipMemcpyDeviceToHost, st));
-    CLM_TRY_HIP(hipStreamSynchronize(st));
+    double rotated = 0;
+    CLM_TRY(read_device_values<int>(st, c->device, ws.count, 1, &rotated));
     converged = rotated == 0;
   }
   if (info) {
