@@ -422,6 +422,11 @@ __global__ void set_info_kernel(int *info, int v) {
 
 // ---- the Taylor route -------------------------------------------------------------------
 constexpr double kTaylorMaxNorm1 = 32.0;
+// the largest workspace a size query asks for on this route's account (it takes 7/3 of the
+// sweeps' in the double types, 8/3 in the single ones): past it, from orders of 23 000
+// (complex64) to 35 000 (FP64), a call whose A, E and sweeps' blocks fit the card might not
+// get this one; it runs the sweeps then
+constexpr size_t kTaylorMaxBytes = size_t(64) << 30;
 
 // the larger; a NaN on either side stays
 __device__ inline double nan_max_(double best, double v) { return v > best || isnan(v) ? v : best; }
@@ -596,7 +601,8 @@ clm_status_t herm_bytes(int n, size_t *bytes) {
   if (bytes == nullptr || n < 1 || n > kMaxDim) return CLM_STATUS_INVALID_VALUE;
   HermWs<work_t<T>> ws;
   HermTaylorWs<T> tw;
-  *bytes = std::max(ws.carve(nullptr, n), tw.carve(nullptr, n));
+  const size_t sweeps = ws.carve(nullptr, n), taylor = tw.carve(nullptr, n);
+  *bytes = taylor > kTaylorMaxBytes ? sweeps : std::max(sweeps, taylor);
   return CLM_STATUS_SUCCESS;
 }
 

@@ -253,9 +253,11 @@ clm_status_t clm_getrs_z(clm_ctx *ctx, clm_stream_t stream, int n, int nrhs,
  * converge within 30 (the result is still written). Synchronizes (the norm, then the
  * exponential's norms or once per sweep).
  * Bad arguments: CLM_STATUS_INVALID_VALUE; a short workspace: CLM_STATUS_ALLOC_FAILED.
- * expm_herm_bufferSize<T> (:97-109): clm_expm_herm_buffer_size_* (the larger of the
- * routes' needs; the Jacobi route's own, three blocks of order n rounded up to 64, is
- * accepted too. The reference holds two blocks and the solver's scratch). */
+ * expm_herm_bufferSize<T> (:97-109): clm_expm_herm_buffer_size_* (the Taylor route's
+ * need up to 64 GiB: 7 blocks of order n in double, 8 for the single-precision types, whose
+ * blocks are double too. The Jacobi route's own, three blocks of order n rounded up to
+ * 64, is accepted everywhere and what the query asks for past 64 GiB; in it every call
+ * takes that route. The reference holds two blocks and the solver's scratch). */
 #define CLM_FILL_MODE_LOWER 0
 #define CLM_FILL_MODE_UPPER 1
 clm_status_t clm_expm_herm_buffer_size_s(int n, size_t *bytes);

@@ -456,3 +456,19 @@ def test_expm_herm_sizes_and_argument_checks():
     assert call(None, None, 1, 4, p, 4, p, 4, None, 1 << 30, None) == ST.INVALID_VALUE
     assert call(None, None, 2, 4, p, 4, p, 4, p, 1 << 30, None) == ST.INVALID_VALUE
     assert call(None, None, 0, 4, p, 4, p, 4, p, 64, None) == ST.ALLOC_FAILED
+
+
+def test_expm_herm_query_never_outgrows_the_card():
+    """a call whose A, E and three sweeps' blocks fit 288 GB gets a workspace that fits it
+    too: past 64 GiB the query asks for the sweeps' blocks alone, not for the Taylor route's"""
+    out = ctypes.c_size_t()
+    card = 288 * 10 ** 9
+    for sfx, size, work in (("s", 4, 8), ("d", 8, 8), ("c", 8, 16), ("z", 16, 16)):
+        f = getattr(L, f"clm_expm_herm_buffer_size_{sfx}")
+        for n in (100, 4096, 16384, 23000, 25000, 33000, 40000, 46340):
+            up = -(-n // 64) * 64
+            sweeps = 3 * up * up * work
+            assert f(n, ctypes.byref(out)) == 0
+            assert sweeps <= out.value <= max(2.7 * sweeps, 1 << 20)
+            if sweeps + 2 * size * n * n <= 0.98 * card:
+                assert out.value + 2 * size * n * n <= card
