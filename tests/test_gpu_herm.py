@@ -1,4 +1,4 @@
-"""GPU: exp(A) for a symmetric / Hermitian A by its eigendecomposition
+"""GPU: exp(A) for a symmetric / Hermitian A through whichever route its norm takes
 (clm_expm_herm_*: the reference's expm_herm, src/expm/expm_herm.cppm:145-199) against
 the oracle's restatement (oracle/herm.py: the uplo triangle, LAPACK's ?syevd/?heevd
 through numpy, U diag(exp(w)) U^H), and the reference's own checks
@@ -10,8 +10,10 @@ through numpy, U diag(exp(w)) U^H), and the reference's own checks
   diagonal's imaginary part filled with NaN (never read);
 * diagonal input: exp of the diagonal to 2 ulp; zero input: the identity exactly;
   degenerate spectra (c I + a rank-2 term);
-* against clm_expm_* (the reference's own oracle for this route);
-* FP32 / complex64 (the sweeps run in double) within 1e-6.
+* against clm_expm_* (the reference's own oracle for this route; up to ||A||_1 = 32 the
+  same chain but for the shift -- the sweeps are compared on such matrices in
+  test_gpu_herm_routes.py);
+* FP32 / complex64 (both routes run in double) within 1e-6.
 """
 import numpy as np
 import pytest
@@ -126,7 +128,7 @@ def test_expm_herm_single(dev, dtype, n):
     a = hermitian(n, 3 * n, CPLX[dtype]).astype(NPC[dtype]).astype(
         np.complex128 if CPLX[dtype] else np.float64)
     e, info = run(a, dtype, dev, "L")
-    # the sweeps run in double: the result is the exact one rounded to single
+    # both routes run in double: the result is the exact one rounded to single
     assert info == 0 and rel(e, oh.expm_herm(a, oh.LOWER)) <= 1e-6
 
 

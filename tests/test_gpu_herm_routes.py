@@ -1,5 +1,6 @@
 """GPU: expm_herm's two routes -- the shifted Taylor exponential up to ||A||_1 = 32, the
-Jacobi sweeps beyond it, for diagonal matrices and in a workspace of the sweeps' size.
+Jacobi sweeps beyond it, for diagonal matrices and in a workspace of the sweeps' size --
+in the four types, with spectra on one side of zero, of one outlier and degenerate.
 
 Both against numpy's eigh (the oracle). Tolerance: eigh's own normwise error bound
 p(n) u ||A||_2 times exp's condition for a Hermitian matrix (1 + ||A||_2), with p(n) = 8 n:
@@ -37,8 +38,8 @@ def _run(a, uplo, dev, nbytes=None):
 
 def _call(a, uplo, dev, nbytes=None, want_info=0):
     n, ld = a.shape[0], a.shape[0] + 1
-    dt = torch.complex128 if np.iscomplexobj(a) else torch.float64
     buf = np.full((n, ld), np.nan, dtype=a.dtype)
+    dt = torch.from_numpy(buf).dtype
     buf[:, :n] = a.T
     other = np.tril(np.ones((n, n), bool), -1) if uplo == "U" else np.triu(np.ones((n, n), bool), 1)
     buf[:, :n].T[other] = np.nan  # never read
@@ -98,3 +99,34 @@ def test_a_value_that_is_not_finite_goes_to_the_sweeps(dev, cplx, n, i, j, bad):
     got, info = _call(a, "U", dev, None, None)
     assert info == want_info
     np.testing.assert_array_equal(got, want)  # NaN where it has NaN
+
+
+def _degenerate(n, cplx, norm):
+    """three eigenvalues only: one of multiplicity n - 2"""
+    rng = np.random.default_rng(n)
+    u = rng.standard_normal((n, 2)) + (1j * rng.standard_normal((n, 2)) if cplx else 0)
+    q, _ = np.linalg.qr(u)
+    h = 0.5 * np.eye(n) + (q * np.array([2.0, -1.5])) @ q.conj().T
+    h = (h + h.conj().T) / 2
+    return h * (norm / np.abs(h).sum(0).max())
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.complex128, np.float32, np.complex64])
+@pytest.mark.parametrize("sweeps", [False, True])
+@pytest.mark.parametrize("kind", ["full", "negative", "degenerate"])
+@pytest.mark.parametrize("n", [2, 31, 64, 150])
+def test_both_routes_on_the_same_matrix(dev, dtype, sweeps, kind, n):
+    """the sweeps through their own workspace at norms the Taylor route takes otherwise. The
+    single types run in double: one rounding of the result, u |E| entrywise, on top"""
+    cplx = np.issubdtype(dtype, np.complexfloating)
+    a = _degenerate(n, cplx, 6.0) if kind == "degenerate" else _spectrum(n, cplx, kind, 6.0, n)
+    a = a.astype(dtype)
+    single = np.finfo(dtype).eps > 1e-10
+    wide = a.astype(np.complex128 if cplx else np.float64)
+    wide = (wide + wide.conj().T) / 2
+    nbytes = _jacobi_bytes(n, 16 if cplx else 8) if sweeps else None
+    for uplo, code in (("U", oh.UPPER), ("L", oh.LOWER)):
+        ref = oh.expm_herm(wide, code)
+        err = np.linalg.norm(_run(a, uplo, dev, nbytes) - ref) / np.linalg.norm(ref)
+        bound = 8 * n * 1.2e-16 * (1 + np.linalg.norm(wide, 2)) + 1e-14
+        assert err <= bound + (np.finfo(dtype).eps if single else 0)
