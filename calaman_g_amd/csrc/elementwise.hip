@@ -325,15 +325,19 @@ hipError_t launch_norm1(hipStream_t stream, int n, const T *A, long lda, real_t<
   return hipGetLastError();
 }
 
-// One workgroup to order 128 (128 KiB of FP64: about the time of a launch to read); above
-// that the columns' sums need the chip, and the maximum and the hand-over share a launch.
+// One workgroup up to 40 KiB of matrix (order 71 in FP64), about the time of a launch to
+// read; above that the columns' sums need the chip, and the maximum and the hand-over share
+// a launch. Whole calls at ||A||_1 = 1, us, three launches / one workgroup / as here: FP64
+// n = 64 91 / 60 / 60, n = 128 108 / 74 / 60, complex128 n = 50 126 / 68 / 68, n = 80 147 /
+// 86 / 76; split FP64 n = 128 80 / 88 / 78 (with the line at order 128, split calls of 80 to
+// 128 were slower than with three launches).
 template <typename T>
 hipError_t launch_norm1_publish(hipStream_t stream, int n, const T *A, long lda, long mstride,
                                 int count, real_t<T> *colsums, double *vals, unsigned *flag,
                                 unsigned seq) {
-  constexpr int kOneWorkgroup = 128;
-  static_assert(kOneWorkgroup <= kRB, "a lane's four registers hold a column");
-  if (n <= kOneWorkgroup) {
+  constexpr size_t kOneWorkgroup = 40 * 1024;
+  static_assert(kOneWorkgroup <= sizeof(T) * kRB * kRB, "a lane's four registers hold a column");
+  if (sizeof(T) * n * n <= kOneWorkgroup) {
     hipLaunchKernelGGL(norm1_publish_kernel<T>, dim3(1), dim3(1024), 0, stream, n, A, lda, mstride,
                        count, vals, flag, seq);
     return hipGetLastError();

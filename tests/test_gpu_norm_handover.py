@@ -1,5 +1,5 @@
-"""GPU: the norms a call plans from (one workgroup up to order 128, the columns' sums and a
-joint maximum above) are bit for bit the 1-norms clm_matrix_norm1_* reports, for the matrix
+"""GPU: the norms a call plans from (one workgroup up to 40 KiB of matrix, the columns' sums
+and a joint maximum above) are bit for bit the 1-norms clm_matrix_norm1_* reports, for the matrix
 and for the powers formed before the plan; a column that is not finite is still seen."""
 import numpy as np
 import pytest
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.float64, torch.complex64, torch.complex128])
-@pytest.mark.parametrize("n", [1, 2, 3, 5, 63, 64, 65, 127, 128, 129, 256, 257, 513])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 50, 51, 63, 64, 65, 71, 72, 101, 102, 127, 128, 129, 256,
+                               257, 513])
 def test_planned_norms_are_the_norms(dev, dt, n):
     gen = torch.Generator(device="cuda").manual_seed(n)
     a = torch.randn((n, n), generator=gen, device=dev, dtype=dt)
