@@ -285,13 +285,17 @@ __global__ void __launch_bounds__(kPanelThreads)
     const T pv = from_lane(prow, 0);
     const bool safe = cabs1(pv) >= min_normal<T>();
     const T rp = safe ? cdiv(ops<T>::from_real(1.0), pv) : ops<T>::zero();
+    if (p != j) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (tid + kPanelThreads * r == p) {  // one lane: its own reads, no other lane's registers
+#pragma unroll
+          for (int c = 0; c < W; ++c) a[r][c] = rows[set][1][c];
+        }
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = tid + kPanelThreads * r;
-      if (i == p && p != j) {  // one lane: its own reads, no other lane's registers
-#pragma unroll
-        for (int c = 0; c < W; ++c) a[r][c] = rows[set][1][c];
-      }
       T l = a[r][0];
       if (nonzero) l = safe ? ops<T>::mul(l, rp) : cdiv(l, pv);
       if (i > j && i < m) blk[i + static_cast<long>(j) * lda] = l;
