@@ -991,9 +991,14 @@ __global__ void __launch_bounds__(threads_of(CFG))
 // the exit once the counter passes `count`.
 // waves per SIMD the registers are held to: a workgroup's barriers and loads hide behind
 // the other workgroups of its CU (1024 complex64 of order 144 on the 32 x 32 tile: 2.25 ms
-// at 3 waves, 1.93 at 4, 2.2 at 5, where the plan's FP64 constants spill in the loop). Real
-// FP32 stops at 3: held to 4 it spills 20 B a lane (856 matrices of order 9 to 85: 501 us at
-// 3 waves, 527 at 4)
+// at 3 waves, 1.93 at 4, 2.2 at 5, where the plan's FP64 constants spill in the loop). It
+// costs 28 to 44 B of spills a lane outside the products' loops, which the full CUs repay:
+// 1024 matrices, us, FP64 on the 32 x 32 tile (36 B) at 3 waves / 4, order 48 686 / 640, 96
+// 1483 / 1126; complex64 there (44 B) order 48 424 / 377, 96 1126 / 923; complex64 on the
+// 64 x 64 tile (28 B) at 2 / 3, order 48 455 / 388, 96 1352 / 1274. A few matrices alone
+// would be 1 to 8% quicker without. Real FP32 stops at 3: held to 4 it spills 20 B (856
+// matrices of order 9 to 85: 501 us at 3 waves, 527 at 4). The 16-wave tiles have 128
+// registers whatever is asked (44 B FP64, 76 B complex64, 276 B complex128).
 template <typename T, int CFG>
 constexpr int min_waves() {
   if (threads_of(CFG) == 1024) return 4;
