@@ -1080,15 +1080,16 @@ constexpr int kDefaultTiles[2][2][2][kBuckets] = {
     {{{0, 1, 3, 3, 1, 2, 4, 4}, {0, 1, 0, 2, 1, 1, 4, 4}},
      {{0, 1, 2, 2, 1, 1, 4, 4}, {0, 1, 0, 1, 0, 1, 1, 1}}}};
 
-// The same for forward plans of few matrices (few_matrices): the longest chain alone is the launch's time, so a matrix takes the tile of the quickest
-// chain whatever that does to a full CU. us, the tiles before per-bucket defaults / default
-// table / this one: 4 FP32 of order 128 408 / 433 / 339, 4 FP64 of order 224 2123 / 2247 /
-// 1512, 64 complex64 of order 48 183 / 201 / 181, 300 of them 239 / 260 / 237, 64 complex128
-// of order 64 389 / 426 / 387. Only while the (type, tile) groups are no more than the
-// streams they run on, or they queue behind each other: 64 of four types, order 4 to 40,
-// 462 us with the default table's 6 groups, 770 with 8.
+// The same for forward plans of few matrices (few_matrices): the longest chain alone is the
+// launch's time, so a matrix takes the tile of the quickest chain whatever that does to a
+// full CU. us, the tiles before per-bucket defaults / default table / this one: 4 FP32 of
+// order 128 408 / 433 / 339, 4 FP64 of order 224 2123 / 2247 / 1512, 64 complex64 of order 48
+// 183 / 201 / 177, 300 of them 239 / 260 / 234, 64 complex128 of order 64 389 / 426 / 387. Only
+// where that makes no more launches than the default table does: with one more, two
+// plans on two streams wait on each other's (two of 64 complex64 of order 4 to 40: 200 us in
+// one group each, 543 in two).
 constexpr int kFewTiles[2][2][kBuckets] = {{{0, 1, 3, 3, 1, 1, 4, 4}, {0, 1, 0, 1, 1, 1, 4, 4}},
-                                           {{0, 1, 2, 2, 1, 1, 4, 4}, {0, 1, 0, 1, 0, 1, 4, 4}}};
+                                           {{0, 1, 2, 2, 1, 1, 4, 4}, {0, 1, 0, 2, 0, 2, 4, 4}}};
 
 void tune_defaults() {
   for (int a = 0; a < 2; ++a)
@@ -1149,67 +1150,49 @@ int few_tile(const clm_batch_entry &e) {
   return (e.n <= 32 * kBuckets ? kFewTiles : g_tune[0])[p][c][bucket_of(e.n)];
 }
 
-// complex FP64 above the 32 x 32 tile: chains that slow each other most on one CU
-bool is_wide(int group) {
-  return group >= group_of(CLM_DTYPE_C128, 0) && group % kTiles != CLM_BATCH_TILE_32;
-}
-
-// How many workgroups a CU may hold, per group (0: as many as fit). The groups of a plan are
-// launched side by side and the device packs each one's workgroups by itself: since a CU's
-// registers hold three chains and more (two at most before, one of complex FP64 above the
-// 32 x 32 tile), a batch of one or two matrices a CU had come to put three on some, whose
-// slowed chains end the launch. So while there is room every matrix has its CU; then two
-// share one, the wide ones still none while there is room; from 2.25 matrices a CU on the
-// device is better left to fill up, except with the shortest chains of all. us, before that
-// change / with it / as claimed here: 400 FP64 of order 4 to 40 373 / 462 / 374, 500 FP32
-// 236 / 295 / 238, 200 FP64 371 / 371 / 312; left to fill up, 600 FP64 of order 33 to 64
-// 664 / 511, held to two 650; held to two, 700 FP64 of order 2 to 12 361 / 419 / 368.
-enum Spread { kAlone, kHalves, kFull };
-Spread spread_groups(const int *group_count, int count, int nmax, int cus, int *per_cu) {
-  constexpr int kTiny = 16;
+// how many of a plan's workgroups a CU has to take when they are spread evenly: 1, 2, or 0
+// for more
+int spread_of(const int *group_count, int cus) {
   // workgroups go round the XCDs, every group from the first one: what an XCD gets at most
-  int wide = 0, other = 0;
-  for (int g = 0; g < kGroups; ++g)
-    (is_wide(g) ? wide : other) += (group_count[g] + kXcds - 1) / kXcds;
+  int most = 0;
+  for (int g = 0; g < kGroups; ++g) most += (group_count[g] + kXcds - 1) / kXcds;
   const int room = cus / kXcds;
-  const Spread how = wide + other <= room             ? kAlone
-                     : wide + (other + 1) / 2 <= room ? kHalves
-                                                      : kFull;
-  const bool two = 4 * count <= 9 * cus || (nmax <= kTiny && count <= 4 * cus);
-  for (int g = 0; g < kGroups; ++g)
-    per_cu[g] = how == kAlone || (how == kHalves && is_wide(g)) ? 1 : how == kHalves || two ? 2 : 0;
-  return how;
+  return most <= room ? 1 : most <= 2 * room ? 2 : 0;
 }
 
-// whether kFewTiles serve a forward plan: a CU for every matrix, or half a one in a single
-// group or beside wide chains; no more groups than lanes; and tuning tables that nobody has
-// changed (the caller holds their mutex)
-bool few_matrices(int count, const clm_batch_entry *entries, int cus, int lanes) {
+// Whether a plan's workgroups claim half a CU's LDS each. The groups of a plan are launched
+// side by side and the device packs each one's workgroups by itself: since a CU's registers
+// hold three chains and more (two at most before), a batch of one or two matrices a CU had
+// come to put three on some, whose slowed chains end the launch. So a CU takes two while that
+// is enough. us, before that change / with it / with the claim: 400 FP64 of order 4 to 40
+// 373 / 462 / 374, 500 FP32 236 / 295 / 238. Past that the device is better left to fill up
+// (530 FP32 of order 16 to 64 241, held to two 306), and so are complex FP64's plans, whose
+// chains above the 32 x 32 tile take a CU to themselves: the others had better crowd. A whole CU
+// for each would be quicker by itself (200 FP64 of order 4 to 40 312 against 371) but shut out
+// a plan on another stream (two of 250 complex64 of order 33 to 64 357 against 247).
+bool claims_half(const int *group_count, int cus) {
+  return std::count(group_count + group_of(CLM_DTYPE_C128, 0), group_count + kGroups, 0) == kTiles &&
+         spread_of(group_count, cus) > 0;
+}
+
+// whether kFewTiles serve a forward plan: one element type; a CU for every matrix, or half a
+// one in a single group; no more groups than the default table makes; and a tuning table
+// that nobody has changed (the caller holds its mutex)
+bool few_matrices(int count, const clm_batch_entry *entries, int cus) {
   if (count > 2 * cus) return false;
-  int used[kGroups] = {}, per_cu[kGroups], nmax = 0;
-  bool all_c64 = true;
+  int used[kGroups] = {}, plain[kGroups] = {};
   for (int i = 0; i < count; ++i) {
     const clm_batch_entry &e = entries[i];
-    nmax = std::max(nmax, e.n);
-    all_c64 &= e.dtype == CLM_DTYPE_C64;
     const int p = precision_of(e.dtype), c = is_complex_code(e.dtype);
-    if (!std::equal(g_tune[0][p][c], g_tune[0][p][c] + kBuckets, kDefaultTiles[0][p][c]))
+    if (e.dtype != entries[0].dtype ||
+        !std::equal(g_tune[0][p][c], g_tune[0][p][c] + kBuckets, kDefaultTiles[0][p][c]))
       return false;
     ++used[group_of(e.dtype, few_tile(e))];
+    ++plain[group_of(e.dtype, kDefaultTiles[0][p][c][bucket_of(e.n)])];
   }
-  int groups = 0;
-  bool wide = false;
-  for (int g = 0; g < kGroups; ++g) {
-    groups += used[g] > 0;
-    wide |= used[g] > 0 && is_wide(g);
-  }
-  const Spread how = spread_groups(used, count, 0, cus, per_cu);
-  // (complex64 whose largest order is 41 to 64: at half a CU each too, 300 of order 16 to 64
-  // 241 / 262 / 229 us; below, one group of the 32 x 32 tile is as quick, above, the larger
-  // orders' default tiles are)
-  const bool c64_to_64 = all_c64 && nmax > 40 && nmax <= 64;
-  return groups <= lanes &&
-         (how == kAlone || (how == kHalves && (groups == 1 || wide || c64_to_64)));
+  const auto groups = [](const int *n) { return kGroups - std::count(n, n + kGroups, 0); };
+  const int per_cu = spread_of(used, cus);
+  return groups(used) <= groups(plain) && (per_cu == 1 || (per_cu == 2 && groups(used) == 1));
 }
 
 // workgroups resident at once on the device for one kernel instantiation
@@ -1228,24 +1211,21 @@ int resident_workgroups(int device) {
   return r;
 }
 
-// LDS a workgroup claims beyond its own `used` bytes to share its CU with one other claimant
-// (per_cu 2) or with none (1); 0: no claim. Why: spread_groups.
-inline size_t lds_claim(int per_cu, size_t used) {
-  constexpr size_t kOfTwo = 56 * 1024, kAlone = 112 * 1024;
-  static_assert(2 * kOfTwo <= 160 * 1024 && 3 * kOfTwo > 160 * 1024 && kAlone + kOfTwo > 160 * 1024,
-                "of a CU's 160 KiB");
-  const size_t want = per_cu == 1 ? kAlone : per_cu == 2 ? kOfTwo : 0;
-  return want > used ? want - used : 0;
+// LDS a workgroup claims beyond its own `used` bytes so that no third fits its CU (claims_half)
+inline size_t lds_claim(bool half, size_t used) {
+  constexpr size_t kHalf = 56 * 1024;
+  static_assert(2 * kHalf <= 160 * 1024 && 3 * kHalf > 160 * 1024, "of a CU's 160 KiB");
+  return half && kHalf > used ? kHalf - used : 0;
 }
 
 template <typename T, int CFG>
 hipError_t launch_group(hipStream_t st, int device, const BatchDesc *desc, int count, int *queue,
-                        char *work, clm_batch_result *results, int per_cu) {
+                        char *work, clm_batch_result *results, bool half) {
   const T *coef = inv_factorials<T>(device);
   if (!coef) return hipErrorInvalidValue;
   const int grid = std::min(count, resident_workgroups<T, CFG>(device));
   hipLaunchKernelGGL((expm_batched_kernel<T, CFG>), dim3(grid), dim3(threads_of(CFG)),
-                     lds_claim(per_cu, lds_bytes<T, CFG>()), st, desc, count, queue, work, results,
+                     lds_claim(half, lds_bytes<T, CFG>()), st, desc, count, queue, work, results,
                      coef);
   return hipGetLastError();
 }
@@ -1313,18 +1293,18 @@ hipError_t launch_adjoint_type(int cfg, hipStream_t st, int device, const BatchD
 
 template <typename T>
 hipError_t launch_type(int cfg, hipStream_t st, int device, const BatchDesc *desc, int count,
-                       int *queue, char *work, clm_batch_result *results, int per_cu) {
+                       int *queue, char *work, clm_batch_result *results, bool half) {
   switch (cfg) {
   case CLM_BATCH_TILE_32:
-    return launch_group<T, CLM_BATCH_TILE_32>(st, device, desc, count, queue, work, results, per_cu);
+    return launch_group<T, CLM_BATCH_TILE_32>(st, device, desc, count, queue, work, results, half);
   case CLM_BATCH_TILE_64:
-    return launch_group<T, CLM_BATCH_TILE_64>(st, device, desc, count, queue, work, results, per_cu);
+    return launch_group<T, CLM_BATCH_TILE_64>(st, device, desc, count, queue, work, results, half);
   case CLM_BATCH_TILE_128x64:
-    return launch_group<T, CLM_BATCH_TILE_128x64>(st, device, desc, count, queue, work, results, per_cu);
+    return launch_group<T, CLM_BATCH_TILE_128x64>(st, device, desc, count, queue, work, results, half);
   case CLM_BATCH_TILE_128:
-    return launch_group<T, CLM_BATCH_TILE_128>(st, device, desc, count, queue, work, results, per_cu);
+    return launch_group<T, CLM_BATCH_TILE_128>(st, device, desc, count, queue, work, results, half);
   default:
-    return launch_group<T, CLM_BATCH_TILE_128W16>(st, device, desc, count, queue, work, results, per_cu);
+    return launch_group<T, CLM_BATCH_TILE_128W16>(st, device, desc, count, queue, work, results, half);
   }
 }
 
@@ -1342,7 +1322,7 @@ struct clm_batch_plan {
   int launch_order[clm::kGroups] = {};   // non-empty groups, costliest first
   int launch_lane[clm::kGroups] = {};    // 0: the caller's stream, i > 0: side[i - 1]
   int num_launch = 0;
-  int per_cu[clm::kGroups] = {};  // workgroups a CU may hold (lds_claim), 0: as many as fit
+  bool half = false;  // workgroups claim half a CU's LDS (claims_half)
   clm::BatchDesc *d_desc = nullptr;    // grouped, each group in decreasing cost
   bool ad = false;                     // records the adjoint tape; backward allowed
   int ckpt = 0;
@@ -1427,13 +1407,10 @@ clm_status_t build_plan(int count, const clm_batch_entry *entries, const int *fo
     const double n = entries[i].n;
     return n * n * n * (is_complex_code(entries[i].dtype) ? 4.0 : 1.0);
   };
-  int nmax = 0;
-  for (int i = 0; i < count; ++i) nmax = std::max(nmax, entries[i].n);
   std::vector<int> cfg(count);
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
-    const bool few =
-        !forced_cfg && !ad && few_matrices(count, entries, cus, 1 + clm_batch_plan::kSide);
+    const bool few = !forced_cfg && !ad && few_matrices(count, entries, cus);
     for (int i = 0; i < count; ++i) {
       const clm_batch_entry &e = entries[i];
       const int p = precision_of(e.dtype), c = is_complex_code(e.dtype);
@@ -1488,8 +1465,9 @@ clm_status_t build_plan(int count, const clm_batch_entry *entries, const int *fo
     plan->group_cost[g] += c;
     longest[g] = std::max(longest[g], c);
   }
+  plan->half = claims_half(plan->group_count, cus);
   // a group whose matrices all have their CU takes as long as its longest chain
-  if (spread_groups(plan->group_count, count, nmax, cus, plan->per_cu) == kAlone)
+  if (spread_of(plan->group_count, cus) == 1)
     std::copy(longest, longest + kGroups, plan->group_cost);
   for (int g = 1; g < kGroups; ++g)
     plan->group_start[g] = plan->group_start[g - 1] + plan->group_count[g - 1];
@@ -1559,13 +1537,13 @@ clm_status_t launch_plan(clm_ctx *ctx, hipStream_t st, const clm_batch_plan *pla
     const int cfg = g % kTiles;
     switch (g / kTiles) {
     case 0: return launch_type<float>(cfg, s, plan->device, desc, count, queue + g, base, results,
-                                  plan->per_cu[g]);
+                                  plan->half);
     case 1: return launch_type<double>(cfg, s, plan->device, desc, count, queue + g, base, results,
-                                  plan->per_cu[g]);
+                                  plan->half);
     case 2: return launch_type<zc>(cfg, s, plan->device, desc, count, queue + g, base, results,
-                                  plan->per_cu[g]);
+                                  plan->half);
     default: return launch_type<zd>(cfg, s, plan->device, desc, count, queue + g, base, results,
-                                  plan->per_cu[g]);
+                                  plan->half);
     }
   });
 }

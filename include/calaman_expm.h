@@ -492,8 +492,8 @@ clm_status_t clm_expm_batched_graph(clm_ctx *ctx, clm_stream_t stream, clm_batch
  * Plans created afterwards use the new table. Its batches are of one order each: for
  * many orders together the default table, which was measured on such batches, can be
  * the faster one (4096 of orders 16 to 256, FP32 and complex64: 15.4 ms, tuned 16.0).
- * While a type's table is the default one, forward plans of few matrices (about one
- * a CU) take tiles chosen for the longest chain instead. */
+ * While a type's table is the default one, forward plans of one type and few matrices
+ * (about one a CU) can take tiles chosen for the longest chain instead. */
 clm_status_t clm_expm_batched_get_tuning(int dtype, int *cfg);
 clm_status_t clm_expm_batched_set_tuning(int dtype, const int *cfg);
 clm_status_t clm_expm_batched_autotune(clm_ctx *ctx, clm_stream_t stream, int dtype, int nmax,

@@ -1,7 +1,7 @@
-"""GPU: batches around one and two matrices a CU, where a plan's tiles and the workgroups a
-CU may hold change (256 CUs: 256 and 512 matrices, 576 above which the device fills up),
-and tiny orders, which are held to two up to four a CU -- of one element type and of
-several. Every member is bit for bit clm_expm_*'s result on the same input.
+"""GPU: batches around one and two matrices a CU, where a plan's tiles and the LDS its
+workgroups claim change (256 CUs in 8 XCDs: 256 and 512 matrices, fewer where several groups
+go round the XCDs), and beyond, of one element type and of several. Every member is bit for
+bit clm_expm_*'s result on the same input; two plans on two streams do not disturb each other.
 """
 import numpy as np
 import pytest
@@ -48,6 +48,27 @@ def test_members_are_the_single_results(dev, types, count, lo, hi):
     for (t, n), (_, _, _, e, _) in zip(picks, entries):
         want = known[t][n][1]
         assert torch.equal(e.view(torch.uint8), want.view(torch.uint8)), (t, n)
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("count,lo,hi", [(200, 33, 64), (260, 4, 40)])
+def test_two_plans_on_two_streams(dev, dtype, count, lo, hi):
+    known = _inputs(dtype, range(lo, hi + 1, 5), dev)
+    orders = list(known)
+    torch.cuda.synchronize()
+    runs = []
+    for k in range(2):
+        picks = [orders[(i + k) % len(orders)] for i in range(count)]
+        entries = [(n, known[n][0], n, torch.empty_like(known[n][0]), n) for n in picks]
+        plan = BatchPlan(entries)
+        runs.append((plan, plan.workspace(), torch.cuda.Stream(), picks, entries))
+    torch.cuda.synchronize()
+    for plan, work, stream, _, _ in runs:
+        assert plan.launch(work, stream=stream) == 0
+    torch.cuda.synchronize()
+    for _, _, _, picks, entries in runs:
+        for n, (_, _, _, e, _) in zip(picks, entries):
+            assert torch.equal(e.view(torch.uint8), known[n][1].view(torch.uint8)), n
 
 
 def test_the_tuner_times_complex128_with_a_cu_to_itself(dev):
